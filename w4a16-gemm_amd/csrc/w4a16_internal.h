@@ -135,6 +135,42 @@ constexpr bool prefill_shape_ok(int cfg, int M, int K) {
 }
 constexpr int prefill_threads(int cfg) { return 64 * kPrefillTable[cfg].waves_m * kPrefillTable[cfg].waves_n; }
 
+// Tiles of prefill_group_kernel_shared (small batches, any K): nb n16 blocks x tm 16-token tiles per
+// workgroup, np producer waves (np / nb chunk pairs per K stage), multiplying waves of cb x ct tiles.
+// One workgroup per CU (LDS).  An auto prefill plan names one in decode_variant when it is the faster
+// kernel for the shape (0: the table's kernel); kernel, grid and block stay those of the table's
+// config, which any caller that clears decode_variant gets.  `us`: measured time of one round of
+// workgroups at K = 4096 (MI355X, weights from HBM).
+struct SharedTile {
+    int nb, tm, cb, ct, np;
+    double us;
+};
+constexpr SharedTile kSharedTable[7] = {
+    {0, 0, 0, 0, 0, 0.0},
+    {2, 1, 1, 1, 8, 8.4},     // 1
+    {2, 2, 2, 1, 8, 10.4},    // 2
+    {4, 1, 2, 1, 12, 11.2},   // 3
+    {4, 2, 2, 2, 12, 14.2},   // 4
+    {4, 3, 2, 3, 8, 17.4},    // 5
+    {4, 4, 2, 2, 8, 19.0},    // 6
+};
+constexpr int kNumSharedTiles = 6;
+constexpr int shared_threads(int id) {
+    return 64 * (kSharedTable[id].np + kSharedTable[id].nb * kSharedTable[id].tm / (kSharedTable[id].cb * kSharedTable[id].ct));
+}
+constexpr int shared_lds_bytes(int id) {                    // two stages of x rows and A fragments
+    return 2 * (2 * (kSharedTable[id].np / kSharedTable[id].nb) * kSharedTable[id].tm * 16 * kLdsRowBytes +
+                kSharedTable[id].np * 4096);
+}
+constexpr int64_t shared_tiles(int id, int M, int N) {
+    return (((int64_t)M + 16 * kSharedTable[id].tm - 1) / (16 * kSharedTable[id].tm)) *
+           ((N / 16 + kSharedTable[id].nb - 1) / kSharedTable[id].nb);
+}
+// x is addressed with 32-bit per-lane byte offsets of up to 63 rows from a 64-bit base.
+constexpr bool shared_shape_ok(int id, int M, int N, int K) {
+    return id >= 1 && id <= kNumSharedTiles && K < (1 << 25) && shared_tiles(id, M, N) < ((int64_t)1 << 31);
+}
+
 // Decode kernel shapes.  A workgroup covers NBW n16 blocks (16*NBW output channels) with WAVES
 // waves splitting its K range.
 //   kind 0: decode_kernel         weights streamed into VGPRs, pipeline depth d chunks, any

@@ -1340,6 +1340,259 @@ prefill_group_kernel(const u4* __restrict__ Wp, const uint16_t* __restrict__ x,
     prefill_tile_out<TM, NB>(acc, m0, nb0_raw, lane, y, ws, counters, M, N, seg, splits, tile);
 }
 
+// Workgroup barrier that orders LDS only: this wave's LDS accesses are complete and its global loads
+// stay in flight (__syncthreads() would drain them).
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
+// Small-batch prefill with shared dequantisation: the tiles of kSharedTable, which w4a16_launch runs
+// in place of the table's kernel when the plan says so (decode_variant of a prefill plan).
+//
+// Few token rows leave each CU a handful of 16 x 16 output tiles, each one MFMA chain over K (the
+// fixed accumulation order).  prefill_group_kernel gives such a tile to one wave that loads,
+// dequantises and multiplies in turn, a barrier per chunk pair: ~0.38 us per pair with one wave per
+// SIMD, most of it latency.  Here a workgroup of one CU covers NB n16 blocks x TM token tiles and
+// splits the work by kind over K stages of P chunk pairs:
+//  * NP producer waves: each stage, wave (block, pair) dequantises one pair of one block (16 bytes of
+//    weights per lane, both nibble parities, so no code is unpacked twice) into MFMA A fragments in
+//    LDS, and stores its share of the x rows in B order; loads run two stages ahead in registers.
+//  * NB TM / (CB CT) multiplying waves, CB blocks x CT token tiles each: per chunk half CB + CT 16-byte
+//    LDS reads and CB CT MFMAs, D steps of reads ahead, at raised priority.
+// Two LDS buffers, one barrier per stage.  Half of the producers store the fragments they dequantised
+// in the previous stage first and dequantise the next ones after (EARLY), the other half dequantise
+// first, so that one half's VALU work overlaps the other half's LDS stores (all in step: 0.77 us
+// per stage of 4 pairs at K = 8192, N = 4096, M = 24; out of step 0.69).
+// Same operands and the same MFMA order per accumulator as every other prefill config (and the same
+// sums of the canonical segments when K > 8192), so the output is bit-identical.  K / 64 may be odd:
+// the last stage of a segment multiplies only its own chunks.  Chunks past the end and rows past M
+// load clamped data that is not multiplied or not stored; blocks past N repeat the last one.
+// Compiler-tracked loads only.  The input pointers are not __restrict__: the compiler would move the
+// prefetches across the memory barriers to just before their use.
+// What bounds it: per stage the chain load wait - dequantisation - LDS - barrier; 2.6 us per launch plus
+// 0.19 us per pair at two blocks x 16 tokens (o, N = K = 4096, M = 24: 11.9 -> 8.4 us; without the
+// MFMAs 7.1, without x 7.0; the bare stream of the weights 5.4); ragged N = 4112, K = 4160 (65
+// chunks), M = 37: 60.8 us (prefill_kernel) -> 11.6.
+template <int NB, int TM, int CB, int CT, int NP>
+__global__ void __launch_bounds__((NP + NB * TM / (CB * CT)) * 64)
+prefill_group_kernel_shared(const u4* Wp, const uint16_t* x, const uint16_t* scales,
+                            int M, int N, int K, int gshift, int groups_m, int seg_chunks, int G, uint16_t* y) {
+    constexpr int PF = 2;                                    // stages of loads in flight (register sets)
+    constexpr int P = NP / NB;                               // chunk pairs per stage
+    constexpr int C = NB * TM / (CB * CT);                   // multiplying waves
+    constexpr int RG = 2 * TM;                               // 8-row groups of x per chunk
+    constexpr int XL = 2 * P * RG / NP;                      // x loads per producer wave and stage
+    constexpr int XCH = TM * 16 * kXRow;                     // LDS bytes of one chunk of x
+    constexpr int XSZ = 2 * P * XCH;
+    constexpr int ASZ = NB * P * 4096;
+    constexpr int BUF = XSZ + ASZ;
+    static_assert(NP % NB == 0 && 2 * P * RG % NP == 0, "work split");
+    __shared__ __attribute__((aligned(16))) char lds[2 * BUF];
+
+    const int lane = threadIdx.x & 63;
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    // Tile order of prefill_group_kernel: each XCD a contiguous range, the token groups of one column
+    // group adjacent.
+    const int G8 = G >> 3;
+    const int bid = blockIdx.x;
+    const int tile = bid < (G8 << 3) ? (bid & 7) * G8 + (bid >> 3) : bid;
+    const int tg = tile % groups_m;
+    const int ng = tile / groups_m;
+    const int KC = K >> 6;
+    const int NBLK = N >> 4;
+    const int m0 = tg * 16 * TM;
+    const int nb0 = ng * NB;
+
+    if (wave >= C) {
+        // Producers: block blk, pair pr of every stage; lane (cc, t, g) holds packed lane 4 g + t of chunk cc.
+        const int pw = wave - C;
+        const int blk = pw / P;                              // this wave's block and pair of every stage
+        const int pr = pw - blk * P;
+        const int nb = min(nb0 + blk, NBLK - 1);
+        const int cc = lane >> 5;
+        const int t = (lane >> 3) & 3;
+        const int g = lane & 7;
+        const char* wbase = reinterpret_cast<const char*>(Wp) + (size_t)nb * KC * 512;
+        const char* sbase = reinterpret_cast<const char*>(scales + (size_t)nb * 16);
+        const char* xbase = reinterpret_cast<const char*>(x + (size_t)m0 * K);
+        const uint32_t woff = (uint32_t)(4 * g + t) * 16;
+        const uint32_t wcc = (uint32_t)cc * 512;
+        const uint32_t soff = (uint32_t)g * 2;
+        const uint32_t scc = gshift ? 0u : (uint32_t)cc * (uint32_t)N * 2u;
+        uint32_t xoff[XL], xlds[XL];
+        int xc[XL];
+#pragma unroll
+        for (int i = 0; i < XL; ++i) {
+            const int id = i * NP + pw;                      // chunk id / RG of the stage, 8-row group id % RG
+            xc[i] = id / RG;
+            const int lr = (id - xc[i] * RG) * 8 + (lane >> 3);
+            const int q = lane & 7;
+            xoff[i] = (uint32_t)(min(m0 + lr, M - 1) - m0) * (uint32_t)K * 2u + (uint32_t)q * 16u;
+            xlds[i] = (uint32_t)(xc[i] * XCH + lr * kXRow + (q >> 2) * 64 + (q & 3) * 4);
+        }
+        Dq de = {0x000F000Fu, h2{(_Float16)1.0f, (_Float16)1.0f}, h2{(_Float16)-1032.0f, (_Float16)-1032.0f}};
+        Dq dodd = {0x00F000F0u, h2{(_Float16)0.0625f, (_Float16)0.0625f}, h2{(_Float16)-72.0f, (_Float16)-72.0f}};
+        asm volatile("" : "+v"(de.mask), "+v"(dodd.mask));
+        auto work = [&](auto early) __attribute__((always_inline)) {
+            constexpr bool EARLY = decltype(early)::value;
+            u4 wq[PF];
+            uint16_t s0[PF], s1[PF];
+            u4 xq[PF][XL];
+            int kl = 0, el = min(seg_chunks, KC);    // cursor of the loads
+            auto issue = [&](auto set) __attribute__((always_inline)) {
+                constexpr int J = decltype(set)::value;
+                const uint32_t mask = kl < KC ? 0xFFFFFFFFu : 0u;      // past the end: one cached address
+                const int kc = min(kl + 2 * pr, KC - 1);
+                const uint32_t two = kc + 1 < KC ? 0xFFFFFFFFu : 0u;
+                wq[J] = *reinterpret_cast<const u4*>(wbase + (size_t)kc * 512 + (size_t)((woff + (wcc & two)) & mask));
+                const char* sb = sbase + (size_t)(kc >> gshift) * N * 2;
+                const size_t so = (soff + (scc & two)) & mask;
+                s0[J] = *reinterpret_cast<const uint16_t*>(sb + so);
+                s1[J] = *reinterpret_cast<const uint16_t*>(sb + 16 + so);
+#pragma unroll
+                for (int i = 0; i < XL; ++i)
+                    xq[J][i] = *reinterpret_cast<const u4*>(xbase + (size_t)min(kl + xc[i], KC - 1) * 128 + (size_t)(xoff[i] & mask));
+                asm volatile("" ::: "memory");
+                kl += 2 * P;
+                if (kl >= el) { kl = el; el = min(el + seg_chunks, KC); }
+            };
+            h8 f[4];
+            auto dequant = [&](auto set) __attribute__((always_inline)) {
+                constexpr int J = decltype(set)::value;
+                const u4 w = wq[J];
+                const h2 se = scale2(s0[J]);
+                const h2 so = scale2(s1[J]);
+                f[0] = dq_frag(w.x, w.y, de, se);
+                f[1] = dq_frag(w.x, w.y, dodd, so);
+                f[2] = dq_frag(w.z, w.w, de, se);
+                f[3] = dq_frag(w.z, w.w, dodd, so);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) asm volatile("" : "+v"(f[i]));
+            };
+            auto store = [&](auto set, int buf) __attribute__((always_inline)) {
+                constexpr int J = decltype(set)::value;
+                char* base = lds + buf * BUF;
+                char* a = base + XSZ + (blk * P + pr) * 4096 + lane * 16;
+#pragma unroll
+                for (int i = 0; i < 4; ++i) *reinterpret_cast<h8*>(a + i * 1024) = f[i];
+#pragma unroll
+                for (int i = 0; i < XL; ++i) {
+                    const u4 v = xq[J][i];
+                    char* b = base + xlds[i];
+                    *reinterpret_cast<uint32_t*>(b) = v.x;
+                    *reinterpret_cast<uint32_t*>(b + 16) = v.y;
+                    *reinterpret_cast<uint32_t*>(b + 32) = v.z;
+                    *reinterpret_cast<uint32_t*>(b + 48) = v.w;
+                }
+                asm volatile("" ::: "memory");
+            };
+            int ks = 0, es = min(seg_chunks, KC);    // cursor of the stored stage
+            static_for<0, PF>([&](auto j) { issue(j); });
+            if constexpr (EARLY) dequant(std::integral_constant<int, 0>{});
+            auto stage = [&](auto j) __attribute__((always_inline)) -> bool {
+                constexpr int J = decltype(j)::value;
+                if constexpr (EARLY) {
+                    store(j, J & 1);
+                    issue(j);
+                    dequant(std::integral_constant<int, (J + 1) % PF>{});
+                } else {
+                    dequant(j);
+                    store(j, J & 1);
+                    issue(j);
+                }
+                lds_barrier();
+                ks += 2 * P;
+                if (ks >= es) { ks = es; es = min(es + seg_chunks, KC); }
+                return ks < KC;
+            };
+            while (stage(std::integral_constant<int, 0>{}) && stage(std::integral_constant<int, 1>{})) {}
+        };
+        if (pw < NP / 2) work(std::true_type{});
+        else work(std::false_type{});
+        return;
+    }
+
+    // Multiplying waves: CB blocks x CT token tiles each.
+    const int kb = lane >> 4;
+    const int li = lane & 15;
+    const int cb0 = wave % (NB / CB) * CB;
+    const int ct0 = wave / (NB / CB) * CT;
+    f4 acc[CT][CB];
+    f4 total[CT][CB];
+#pragma unroll
+    for (int t = 0; t < CT; ++t)
+#pragma unroll
+        for (int b = 0; b < CB; ++b) { acc[t][b] = f4{0.f, 0.f, 0.f, 0.f}; total[t][b] = f4{0.f, 0.f, 0.f, 0.f}; }
+    // Step i = 4 p + 2 cc + h of a stage: CB A fragments, CT B operands, CB CT MFMAs.  The schedule
+    // below keeps the reads of D steps ahead of the MFMAs (the compiler counts the waits).
+    constexpr int D = 12 / (CB + CT) < 4 * P ? 12 / (CB + CT) : 4 * P;
+    const char* xr0 = lds + (ct0 * 16 + li) * kXRow + kb * 16;
+    const char* ar0 = lds + XSZ + cb0 * P * 4096 + (li >> 3) * 1024 + kb * 128 + (li & 7) * 16;
+    auto step = [&](const char* xr, const char* ar) __attribute__((always_inline)) {
+        h8 fa[CB], fb[CT];
+#pragma unroll
+        for (int i = 0; i < CB; ++i) fa[i] = *reinterpret_cast<const h8*>(ar + i * P * 4096);
+#pragma unroll
+        for (int j = 0; j < CT; ++j) fb[j] = *reinterpret_cast<const h8*>(xr + j * 16 * kXRow);
+#pragma unroll
+        for (int j = 0; j < CT; ++j)
+#pragma unroll
+            for (int i = 0; i < CB; ++i) acc[j][i] = mfma16x16x32(fa[i], fb[j], acc[j][i]);
+    };
+    __builtin_amdgcn_s_setprio(2);
+    int ks = 0, es = min(seg_chunks, KC);
+    int off = 0;
+    bool first = true;
+    while (ks < KC) {
+        lds_barrier();
+        const int left = es - ks;
+        const char* xr = xr0 + off;
+        const char* ar = ar0 + off;
+        if (left >= 2 * P) {
+            static_for<0, 4 * P>([&](auto i) {
+                constexpr int I = decltype(i)::value, c = I / 2, h = I & 1;
+                step(xr + c * XCH + h * 64, ar + (c >> 1) * 4096 + (c & 1) * 512 + h * 2048);
+            });
+            __builtin_amdgcn_sched_group_barrier(0x100, D * (CB + CT), 0);
+            static_for<0, 4 * P>([&](auto i) {
+                __builtin_amdgcn_sched_group_barrier(0x008, CB * CT, 0);
+                if constexpr (decltype(i)::value + D < 4 * P) __builtin_amdgcn_sched_group_barrier(0x100, CB + CT, 0);
+            });
+        } else {
+#pragma unroll 1
+            for (int c = 0; c < left; ++c) {
+                step(xr + c * XCH, ar + (c >> 1) * 4096 + (c & 1) * 512);
+                step(xr + c * XCH + 64, ar + (c >> 1) * 4096 + (c & 1) * 512 + 2048);
+            }
+        }
+        off = BUF - off;
+        ks += 2 * P;
+        if (ks >= es) {
+            ks = es;
+            es = min(es + seg_chunks, KC);
+#pragma unroll
+            for (int t = 0; t < CT; ++t)
+#pragma unroll
+                for (int b = 0; b < CB; ++b) {
+                    total[t][b] = first ? acc[t][b] : total[t][b] + acc[t][b];
+                    acc[t][b] = f4{0.f, 0.f, 0.f, 0.f};
+                }
+            first = false;
+        }
+    }
+
+#pragma unroll
+    for (int b = 0; b < CB; ++b) {
+        const int nb = nb0 + cb0 + b;
+        if (nb >= NBLK) break;
+#pragma unroll
+        for (int t = 0; t < CT; ++t) {
+            const int m = m0 + (ct0 + t) * 16 + li;
+            if (m < M) *reinterpret_cast<u2*>(y + (size_t)m * N + (size_t)nb * 16 + 4 * kb) = pack_f16x4(total[t][b]);
+        }
+    }
+}
+
 // ------------------------------------------------------------------------------------ launch
 
 // Wide prefill configs (kind 1) live in their own translation unit (w4a16_prefill_wide.hip),
@@ -1452,6 +1705,30 @@ static hipError_t launch_cached(unsigned grid, unsigned block, hipStream_t st, A
     }
     void* params[] = {static_cast<void*>(&args)...};
     return hipModuleLaunchKernel(f, grid, 1, 1, block, 1, 1, 0, st, params, nullptr);
+}
+
+template <int ID>
+static hipError_t launch_shared_id(const w4a16_plan& p, const u4* Wp, const uint16_t* x, const uint16_t* s, uint16_t* y,
+                                   hipStream_t st) {
+    constexpr SharedTile t = kSharedTable[ID];
+    const int groups_m = (p.M + 16 * t.tm - 1) / (16 * t.tm);
+    const int grid = (int)shared_tiles(ID, p.M, p.N);
+    return launch_cached<prefill_group_kernel_shared<t.nb, t.tm, t.cb, t.ct, t.np>>(
+        (unsigned)grid, (unsigned)shared_threads(ID), st, Wp, x, s, (int)p.M, (int)p.N, (int)p.K, p.G == 128 ? 1 : 0,
+        groups_m, prefill_segment_chunks(p.K >> 6), grid, y);
+}
+
+static hipError_t launch_prefill_shared(const w4a16_plan& p, const u4* Wp, const uint16_t* x, const uint16_t* s,
+                                        uint16_t* y, hipStream_t st) {
+    switch (p.decode_variant) {
+        case 1: return launch_shared_id<1>(p, Wp, x, s, y, st);
+        case 2: return launch_shared_id<2>(p, Wp, x, s, y, st);
+        case 3: return launch_shared_id<3>(p, Wp, x, s, y, st);
+        case 4: return launch_shared_id<4>(p, Wp, x, s, y, st);
+        case 5: return launch_shared_id<5>(p, Wp, x, s, y, st);
+        case 6: return launch_shared_id<6>(p, Wp, x, s, y, st);
+        default: return hipErrorInvalidValue;
+    }
 }
 
 template <int V>
@@ -1645,6 +1922,7 @@ int check_plan(const w4a16_plan& p) {
     if (segs > 1 && ((int64_t)p.counter_slots < tiles ||
                      p.workspace_bytes < (uint64_t)segs * p.M * p.N * sizeof(float)))
         return W4A16_ERR_WORKSPACE;
+    if (p.decode_variant && !shared_shape_ok(p.decode_variant, p.M, p.N, p.K)) return W4A16_ERR_INVALID;
     return W4A16_OK;
 }
 }  // namespace
@@ -1670,6 +1948,8 @@ extern "C" int w4a16_launch(const w4a16_plan* plan, const int32_t* Wp, const uin
         float* ws = reinterpret_cast<float*>(workspace);
         int* cnt = reinterpret_cast<int*>(counters);
         e = launch_decode(p, wp, x, scales, y, ws, cnt, st);
+    } else if (p.decode_variant) {
+        e = launch_prefill_shared(p, wp, x, scales, y, st);
     } else {
         switch (p.kernel) {
             case 1: e = launch_prefill<1>(p, wp, x, scales, y, reinterpret_cast<float*>(workspace), counters, st); break;

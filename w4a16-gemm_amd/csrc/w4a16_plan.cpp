@@ -226,6 +226,45 @@ int prefill_select(int M, int N, int K, const w4a16_device_limits& lim) {
     return best;
 }
 
+// The shared-dequantisation tile (kSharedTable) to run instead of the auto config, or 0.  Measured on
+// MI355X over N = 256..28672, K = 1024..14400, M = 1..1024 (graph-timed, weights from HBM):
+//  * one K chain (K <= 8192): the narrowest tile whose workgroups fit one per CU.  It beats the auto
+//    config on every such shape, e.g. K = 4096: N = 4096, M = 24 8.4 vs 11.9 us (token groups of 16),
+//    M = 64 10.5 vs 12.1, M = 96 13.5 vs 15.7, M = 192 15.7 vs 18.8, M = 256 18.1 vs 19.9; N = 14336,
+//    M = 32 14.8 vs 16.4, M = 48 17.3 vs 21.2; N = 6144, M = 128 17.9 vs 18.9; in two rounds it loses
+//    (N = 28672, M = 32: 26 vs 21.6).  Not below K = 1024, where the launch of its larger workgroups
+//    outweighs the shorter chain, and the 64-channel tile only from K = 2048 (N = 10256, M = 5,
+//    K = 1024: 5.16 vs 4.79).
+//  * longer K: the token groups run the segments on workgroups of their own and are as fast (K = 14336,
+//    N = 4096, M = 32: 18.2 vs 18.6); kept.
+//  * K / 64 odd: the ring, token-group and wide kernels do not take it, prefill_kernel does at
+//    ~0.8 us per chunk, so the cheapest tile by rounds x us (scaled with K) while that is below 1.1 us
+//    per chunk: N = 4112, K = 4160, M = 37 11.6 vs 60.8 us, M = 513 47 vs 72; N = 28672, K = 14400,
+//    M = 1 65 vs 229; at M = 1024, N = 4112, K = 4160 both take 88.
+int shared_select(int M, int N, int K, const w4a16_device_limits& lim) {
+    const int64_t cus = lim.cu_count > 0 ? lim.cu_count : 1;
+    const int KC = K / 64;
+    auto ok = [&](int id) {
+        return shared_shape_ok(id, M, N, K) && shared_lds_bytes(id) <= lim.lds_bytes_per_block &&
+               shared_threads(id) <= lim.max_threads_per_block;
+    };
+    if (KC % 2 == 0) {
+        if (prefill_segments(KC) > 1 || KC < 16) return 0;
+        for (int id = 1; id <= kNumSharedTiles; ++id)
+            if (ok(id) && shared_tiles(id, M, N) <= cus) return id == 3 && KC < 32 ? 0 : id;
+        return 0;
+    }
+    int best = 0;
+    double best_us = 1.1 * KC;
+    for (int id = 1; id <= kNumSharedTiles; ++id) {
+        if (!ok(id)) continue;
+        const double rounds = (double)((shared_tiles(id, M, N) + cus - 1) / cus);
+        const double us = rounds * (2.6 + (kSharedTable[id].us - 2.6) * KC / 64.0);
+        if (us < best_us) { best_us = us; best = id; }
+    }
+    return best;
+}
+
 }  // namespace
 
 extern "C" void w4a16_set_last_error(const char* msg) { g_last_error = msg ? msg : ""; }
@@ -463,8 +502,17 @@ extern "C" int w4a16_plan_create(const w4a16_problem* prob, int variant, const w
                          out.slab_chunks, splits, out.grid);
     } else {
         int cfg = v;                                          // 1..4 forced, or -1 = auto
+        int shared = 0;
         if (cfg < 0) {
-            if (const char* o = std::getenv("W4A16_PREFILL")) {   // tuning override: prefill config id
+            const char* o = std::getenv("W4A16_PREFILL");
+            const char* so = std::getenv("W4A16_PREFILL_SHARED");     // tuning override: shared tile id, 0 = none
+            const int sid = so ? std::atoi(so) : -1;
+            if (sid > 0 && shared_shape_ok(sid, M, N, K) && shared_lds_bytes(sid) <= lim->lds_bytes_per_block &&
+                shared_threads(sid) <= lim->max_threads_per_block)
+                shared = sid;
+            else if (sid < 0 && !o)
+                shared = shared_select(M, N, K, *lim);
+            if (o) {   // tuning override: prefill config id
                 const int oc = std::atoi(o);
                 if (oc >= 1 && oc <= kNumPrefillTable && prefill_occupancy(oc, *lim) > 0 && prefill_shape_ok(oc, M, K)) cfg = oc;
             }
@@ -484,9 +532,10 @@ extern "C" int w4a16_plan_create(const w4a16_problem* prob, int variant, const w
         if (kPrefillTable[cfg].kind >= 2 && segs > 1 && tiles_of(cfg) > kMaxCounterSlots) cfg = 4;
         if (!fill_prefill_plan(cfg, &out))
             return fail(W4A16_ERR_INVALID, err, errlen, "M too large for prefill config %d", cfg);
+        out.decode_variant = shared;
         if (debug_enabled())
-            std::fprintf(stderr, "prefill dispatch G=%d M=%d N=%d K=%d cfg=%d occ=%d tiles=%d\n",
-                         G, M, N, K, cfg, prefill_occupancy(cfg, *lim), out.grid);
+            std::fprintf(stderr, "prefill dispatch G=%d M=%d N=%d K=%d cfg=%d occ=%d tiles=%d shared=%d\n",
+                         G, M, N, K, cfg, prefill_occupancy(cfg, *lim), out.grid, shared);
     }
     *plan = out;
     return W4A16_OK;

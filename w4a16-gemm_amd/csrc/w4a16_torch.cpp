@@ -294,7 +294,10 @@ py::dict w4a16_plan_info(int64_t M, int64_t N, int64_t K, int64_t G, int64_t var
                                        : tmpl(kinds[c.kind], {c.nbw, c.waves, c.d});
     } else {
         const w4a16::PrefillTile& t = w4a16::kPrefillTable[plan.kernel];
-        if (t.kind == 2)
+        if (plan.decode_variant) {
+            const w4a16::SharedTile& h = w4a16::kSharedTable[plan.decode_variant];
+            d["kernel_name"] = tmpl("prefill_group_kernel_shared", {h.nb, h.tm, h.cb, h.ct, h.np});
+        } else if (t.kind == 2)
             d["kernel_name"] = tmpl("prefill_stream_kernel", {t.bm / 16, t.depth});
         else if (t.kind == 3)
             d["kernel_name"] = tmpl("prefill_group_kernel", {t.bm / 16, t.depth, t.waves_n, t.bn / (16 * t.waves_n)});
