@@ -166,7 +166,7 @@ int w4a16_quantize_pack(const void* W, int w_is_fp32, int64_t N, int64_t K, int6
  * acc is the exact sum of wv(n, k) * A[k] rounded once to fp32 (the reference sums in fp32 in k
  * order; the two differ by that order's rounding error only).  Inf and NaN inputs give the IEEE
  * result of the sum.  K % 8 == 0, 0 <= K <= W4A16_GEMV_MAX_K; W 4-byte aligned, the others 2-byte
- * aligned (16-byte alignment of W with K % 32 == 0, and of A, selects wider loads).  Asynchronous
+ * aligned (16-byte alignment of A selects wider loads).  Asynchronous
  * on `stream`, allocates nothing.  Returns W4A16_OK, W4A16_ERR_INVALID (message via
  * w4a16_last_error) or W4A16_ERR_HIP. */
 int w4a16_gemv(const int32_t* W, const uint16_t* A, const uint16_t* sW, const uint16_t* zW, uint16_t* C,

@@ -26,6 +26,16 @@
 // 16, lane / 16) loads 16 bytes of row r per superchunk: the 32 weights at k = 128p + 32g .. +31,
 // two MFMAs' worth (k offsets 0..15 and 16..31 of its group).  The MFMA output tiles of the 8
 // waves (row 4g + i, digit r in lane (r, g), element i) are summed in LDS (exact integers).
+//
+// The A operand holds the nibbles offset by 8 (n ^ 8 = wv + 8, unsigned, two operations per dword
+// instead of four), and one more MFMA per B operand with a weight of one in every row gives the digit
+// sums, so P_j = sum_k (wv + 8) L_j - 8 sum_k L_j (below 15 * 128 * 2^20 < 2^31 before the
+// subtraction).
+//
+// What bounds it: the launch and the first round trip at small N K (K = N = 4096: 4.7 us, 4.9 before this
+// loop), the weight stream at large (N = 28672, K = 8192: 31.2 us, 3.8 TB/s, 35.0 before).  Rows that are
+// not whole 16-byte units cost what others do: N = 9184, K = 888 4.6 us against 11.6 with 4-byte loads,
+// N = 20000, K = 2000 7.6 against 19.1; two segments in flight: N = 4096, K = 14336 10.3 against 13.9.
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -39,6 +49,11 @@ namespace w4a16 {
 
 namespace {
 
+// Workgroup barrier that orders LDS only (global loads stay in flight).
+__device__ __forceinline__ void lds_barrier() {
+    asm volatile("s_waitcnt lgkmcnt(0)\n\ts_barrier" ::: "memory");
+}
+
 typedef int32_t i4v __attribute__((ext_vector_type(4)));
 
 constexpr int kRows = 16;                  // rows per MFMA row tile
@@ -49,23 +64,22 @@ constexpr int kSuper = 128;                // k per superchunk (16 bytes of a ro
 constexpr int kDigits = 6;                 // base-256 digits of a * 2^24
 constexpr int kSuperBytes = 2 * 4 * kDigits * 16;   // table bytes per superchunk (768)
 constexpr int kPerWave = kSeg / kSuper / kWaves;   // superchunks per wave and segment (4)
-constexpr uint64_t kDigitBias = 0x808080808080ull;  // 128 * sum_j 256^j
 
 static_assert(kSeg % (kSuper * kWaves) == 0, "segment must split evenly over the waves");
 static_assert(kSeg / 8 == kThreads, "the table build gives each thread one 8-k unit");
 
-// a * 2^24 + kDigitBias for a finite fp16 a (callers pass 0 for inputs that must count as 0).
-// Branch-free: the hidden bit is min(e, 1), the mantissa is shifted by e - min(e, 1), and the
-// sign is applied as (mag ^ s) - s = (mag ^ s) + (s & 1) with s = 0 or all ones, folded into the
-// bias.
-__device__ __forceinline__ uint64_t biased_fixed(uint32_t h) {
-    const uint32_t e = (h >> 10) & 31u;
-    const uint32_t hid = min(e, 1u);
-    const uint32_t mant = (h & 1023u) | (hid << 10);
-    const uint64_t mag = (uint64_t)mant << (e - hid);
-    const uint32_t s = 0u - ((h >> 15) & 1u);
-    const uint64_t sx = ((uint64_t)s << 32) | s;
-    return (mag ^ sx) + (kDigitBias + (s & 1u));
+// The balanced digits of a finite fp16 a (callers pass 0 for inputs that must count as 0), split at
+// 2^24: a * 2^24 = hi * 2^24 + lo with hi an integer and lo in [-0x808080, 0x7F7F7F], so lo gives
+// digits 0..2 and hi digits 3..5.  hi = rne(a + 1/510): the window of lo is off centre by 1/510, and
+// the sum stays on the right side of it for every fp16 value (checked exhaustively, see the tests).
+// Adding 2^23 + 0x408080 rounds to an integer and leaves hi + 0x408080 in the low mantissa bytes;
+// lo + 0x808080 is formed exactly by one fma.  Seven fp32 operations per value.
+constexpr float kHiMagic = 8388608.0f + 4227200.0f;          // 2^23 + 0x408080
+constexpr float kHiBias = 0.00196f;                          // about 1/510
+__device__ __forceinline__ void split_fixed(float f, uint32_t& lo, uint32_t& hi) {
+    const float m = (f + kHiBias) + kHiMagic;
+    hi = __builtin_bit_cast(uint32_t, m);
+    lo = (uint32_t)__builtin_fmaf(f - (m - kHiMagic), 16777216.0f, 8421504.0f);
 }
 
 // 4x4 byte transpose: out[j] byte i = byte j of in[i] (v_perm_b32 picks bytes of {src0, src1},
@@ -81,28 +95,22 @@ __device__ __forceinline__ void byte_transpose(const uint32_t (&in)[4], uint32_t
     out[3] = __builtin_amdgcn_perm(u23h, u01h, 0x07060302u);
 }
 
-// Digit dwords of four biased values: d[j] byte i = digit j of value i as a signed byte
-// (the byte of X + kDigitBias minus 128, i.e. XOR 0x80), j = 0..5.
-__device__ __forceinline__ void digit_dwords(const uint64_t (&v)[4], uint32_t (&d)[kDigits]) {
-    const uint32_t lo[4] = {(uint32_t)v[0], (uint32_t)v[1], (uint32_t)v[2], (uint32_t)v[3]};
+// Digit dwords of four values: d[j] byte i = digit j of value i as a signed byte.  The bytes of lo
+// are the digits plus 128 (XOR 0x80); of hi likewise, the third plus 64 (0x3F..0x41).
+__device__ __forceinline__ void digit_dwords(const uint32_t (&lo)[4], const uint32_t (&hi)[4], uint32_t (&d)[kDigits]) {
     uint32_t t[4];
     byte_transpose(lo, t);
 #pragma unroll
-    for (int j = 0; j < 4; ++j) d[j] = t[j] ^ 0x80808080u;
-    const uint32_t h0 = (uint32_t)(v[0] >> 32), h1 = (uint32_t)(v[1] >> 32);
-    const uint32_t h2 = (uint32_t)(v[2] >> 32), h3 = (uint32_t)(v[3] >> 32);
-    const uint32_t v01 = __builtin_amdgcn_perm(h1, h0, 0x05010400u);
-    const uint32_t v23 = __builtin_amdgcn_perm(h3, h2, 0x05010400u);
-    d[4] = __builtin_amdgcn_perm(v23, v01, 0x05040100u) ^ 0x80808080u;
-    d[5] = __builtin_amdgcn_perm(v23, v01, 0x07060302u) ^ 0x80808080u;
+    for (int j = 0; j < 3; ++j) d[j] = t[j] ^ 0x80808080u;
+    byte_transpose(hi, t);
+    d[3] = t[0] ^ 0x80808080u;
+    d[4] = t[1] ^ 0x80808080u;
+    d[5] = (t[2] + 0x40404040u) ^ 0x80808080u;
 }
 
-// Signed bytes of the even (shift 0) or odd (shift 4) nibbles of a word: nibble n becomes
-// n - 16 * (n >= 8).  With u = n ^ 8 (in 0..15), (u + 0x78) ^ 0x80 is that value as a byte and
-// no byte carries into the next.
-__device__ __forceinline__ uint32_t signed_nibbles(uint32_t w, int shift) {
-    const uint32_t u = ((w ^ 0x88888888u) >> shift) & 0x0F0F0F0Fu;
-    return (u + 0x78787878u) ^ 0x80808080u;
+// The even (shift 0) or odd (shift 4) nibbles of a word as bytes offset by 8: n ^ 8 = wv + 8.
+__device__ __forceinline__ uint32_t offset_nibbles(uint32_t w, int shift) {
+    return ((w >> shift) ^ 0x08080808u) & 0x0F0F0F0Fu;
 }
 
 // IEEE class of the non-finite terms of row n (only called when A holds inf or NaN).
@@ -121,22 +129,26 @@ __device__ int nonfinite_class(const uint32_t* __restrict__ wrow, const uint16_t
     return nan || (pos && neg) ? 3 : pos ? 1 : neg ? 2 : 0;
 }
 
-// WVEC: rows are 16-byte aligned (W 16-byte aligned and K % 32 == 0), one 16-byte load per lane
-// and superchunk; otherwise four 4-byte loads.  Loads past the row's end are redirected to its
-// first word: their digits are zero (the table is zero for k >= K), so they add nothing.
+// Lanes load 16 bytes of their row at any 4-byte alignment (K % 8 == 0 makes rows whole words; the
+// hardware takes dword-aligned 16-byte loads).  A lane whose 4 words cross the row's end loads the
+// row's last 4 words and shifts them down when they are used; lanes past the end multiply zero digits
+// (the table is zero for k >= K), so what they load does not matter.  NARROW: rows of fewer than 4 words.
 // XVEC: A is 16-byte aligned (one 16-byte load per 8 values); otherwise eight 2-byte loads.
 //
-// Segments are double-buffered: the A values and weights of segment s + 1 are requested before
-// the MFMAs of segment s, so their latency overlaps that work.  Every load is issued
-// unconditionally (clamped addresses) so the compiler's waits count exactly the loads in flight.
-// RT: row tiles of 16 per workgroup.  Each digit-table B operand feeds RT MFMAs, so the A
+// MULTI (K > 4096): two segments are in flight (the loads of segment s + 2 are issued once segment s is
+// multiplied) and two digit tables leave one barrier per segment, which waits for LDS only.  Every load is issued
+// unconditionally (clamped addresses) so the compiler's waits count exactly the loads in flight; the
+// pointers are not __restrict__, or it would move the loads down to their use.
+// RT: row tiles of 16 per workgroup.  Each digit-table B operand feeds RT + 1 MFMAs, so the A
 // conversion (done once per workgroup and segment) is shared by 16 RT rows.
-template <bool WVEC, bool XVEC, int RT>
+typedef u4 u4_a4 __attribute__((aligned(4)));
+
+template <bool NARROW, bool XVEC, int RT, bool MULTI>
 __global__ void __launch_bounds__(kThreads)
-gemv_kernel(const uint32_t* __restrict__ W, const uint16_t* __restrict__ A, const uint16_t* __restrict__ sW,
-            const uint16_t* __restrict__ zW, uint16_t* __restrict__ C, int N, int K) {
+gemv_kernel(const uint32_t* W, const uint16_t* A, const uint16_t* sW, const uint16_t* zW, uint16_t* C, int N, int K) {
     constexpr int ROWS = kRows * RT;
-    __shared__ __align__(16) uint8_t table[kSeg / kSuper * kSuperBytes];
+    constexpr int kTable = kSeg / kSuper * kSuperBytes;
+    __shared__ __align__(16) uint8_t table[(MULTI ? 2 : 1) * kTable];
     __shared__ int32_t part[kWaves][ROWS][8];
     const int tid = threadIdx.x;
     const int lane = tid & 63;
@@ -144,10 +156,11 @@ gemv_kernel(const uint32_t* __restrict__ W, const uint16_t* __restrict__ A, cons
     const int r = lane & 15, g = lane >> 4;
     const int row0 = blockIdx.x * ROWS;
     const int kw = K >> 3;                                   // words per row
-    const uint32_t* __restrict__ wrow[RT];
+    const char* wbase = reinterpret_cast<const char*>(W + (size_t)row0 * kw);
+    uint32_t woff[RT];                                       // bytes from wbase, below 32 * 2^19
 #pragma unroll
-    for (int t = 0; t < RT; ++t) wrow[t] = W + (size_t)min(row0 + kRows * t + r, N - 1) * kw;
-    i4v acc[RT];
+    for (int t = 0; t < RT; ++t) woff[t] = (uint32_t)(min(row0 + kRows * t + r, N - 1) - row0) * (uint32_t)kw * 4u;
+    i4v acc[RT], sums = {0, 0, 0, 0};
 #pragma unroll
     for (int t = 0; t < RT; ++t) acc[t] = i4v{0, 0, 0, 0};
     int nonfinite = 0;
@@ -157,10 +170,12 @@ gemv_kernel(const uint32_t* __restrict__ W, const uint16_t* __restrict__ A, cons
         nsc = (min(kSeg, K - seg) + kSuper - 1) / kSuper;
         per = (nsc + kWaves - 1) / kWaves;
     };
-    // Request the A values of this thread's 8-k unit and this wave's weights for segment `seg`.
+    // Request the A values of this thread's 8-k unit and this wave's weights for segment `seg` (past
+    // the end, MULTI: one cached address, unused).
     auto issue = [&](int seg, u4& xa, u4 (&wq)[RT][kPerWave]) {
+        const uint32_t live = !MULTI || seg < K ? 0xFFFFFFFFu : 0u;
         int nsc, per;
-        shape(seg, nsc, per);
+        shape(min(seg, K - 1), nsc, per);
         const int k0 = seg + 8 * tid;
         const uint16_t* src = A + (k0 < K ? k0 : 0);
         if constexpr (XVEC) {
@@ -177,20 +192,22 @@ gemv_kernel(const uint32_t* __restrict__ W, const uint16_t* __restrict__ A, cons
             const int wi = ((seg + p * kSuper) >> 3) + 4 * g;   // first word of the lane's 32 weights
 #pragma unroll
             for (int t = 0; t < RT; ++t) {
-                if constexpr (WVEC) {
-                    wq[t][i] = *reinterpret_cast<const u4*>(wrow[t] + (wi + 4 <= kw ? wi : 0));
-                } else {
+                if constexpr (NARROW) {
                     uint32_t d[4];
 #pragma unroll
-                    for (int e = 0; e < 4; ++e) d[e] = wrow[t][wi + e < kw ? wi + e : 0];
+                    for (int e = 0; e < 4; ++e)
+                        d[e] = *reinterpret_cast<const uint32_t*>(wbase + woff[t] + 4u * (uint32_t)min(wi + e, kw - 1));
                     wq[t][i] = u4{d[0], d[1], d[2], d[3]};
+                } else {
+                    wq[t][i] = *reinterpret_cast<const u4_a4*>(wbase + ((woff[t] + 4u * (uint32_t)min(wi, kw - 4)) & live));
                 }
             }
         }
+        asm volatile("" ::: "memory");
     };
-    // Digits of this thread's unit into the table (units past the segment's superchunks are
+    // Digits of this thread's unit into a table (units past the segment's superchunks are
     // never read; units past K write zero digits).
-    auto build = [&](int seg, const u4& xa) {
+    auto build = [&](int seg, const u4& xa, uint8_t* tab) {
         int nsc, per;
         shape(seg, nsc, per);
         const int u = tid;
@@ -214,65 +231,85 @@ gemv_kernel(const uint32_t* __restrict__ W, const uint16_t* __restrict__ A, cons
                          ((ee >> 16) == 0x7C00u ? 0x0000FFFFu : 0xFFFFFFFFu);
             }
         }
-        uint64_t ve[4], vo[4];                               // k offsets 0, 2, 4, 6 and 1, 3, 5, 7
+        uint32_t le[4], he[4], lo[4], ho[4];                 // k offsets 0, 2, 4, 6 and 1, 3, 5, 7
 #pragma unroll
-        for (int i = 0; i < 8; ++i) (i & 1 ? vo : ve)[i >> 1] = biased_fixed((hw[i >> 1] >> (16 * (i & 1))) & 0xFFFFu);
+        for (int i = 0; i < 4; ++i) {
+            split_fixed((float)__builtin_bit_cast(_Float16, (uint16_t)(hw[i] & 0xFFFFu)), le[i], he[i]);
+            split_fixed((float)__builtin_bit_cast(_Float16, (uint16_t)(hw[i] >> 16)), lo[i], ho[i]);
+        }
         uint32_t de[kDigits], dd[kDigits];
-        digit_dwords(ve, de);
-        digit_dwords(vo, dd);
+        digit_dwords(le, he, de);
+        digit_dwords(lo, ho, dd);
         const int p = u >> 4, rr = (u & 15) * 8;             // superchunk, k offset in it
         const int gg = rr >> 5, m = (rr >> 4) & 1, h = (rr >> 3) & 1;
-        uint8_t* dst = table + p * kSuperBytes + ((m * 4 + gg) * kDigits) * 16 + 8 * h;
+        uint8_t* dst = tab + p * kSuperBytes + ((m * 4 + gg) * kDigits) * 16 + 8 * h;
 #pragma unroll
         for (int j = 0; j < kDigits; ++j) *reinterpret_cast<uint2*>(dst + 16 * j) = uint2{de[j], dd[j]};
     };
-    auto multiply = [&](int seg, const u4 (&wq)[RT][kPerWave]) {
+    auto multiply = [&](int seg, const u4 (&wq)[RT][kPerWave], const uint8_t* tab) {
         int nsc, per;
         shape(seg, nsc, per);
+        const i4v ones = {0x01010101, 0x01010101, 0x01010101, 0x01010101};
 #pragma unroll
         for (int i = 0; i < kPerWave; ++i) {
             const int p = wave * per + i;
             if (i >= per || p >= nsc) break;
+            i4v b[2];
 #pragma unroll
             for (int m = 0; m < 2; ++m) {
-                i4v b = {0, 0, 0, 0};
-                if (r < kDigits) {
-                    const u4 t = *reinterpret_cast<const u4*>(table + p * kSuperBytes + ((m * 4 + g) * kDigits + r) * 16);
-                    b = i4v{(int32_t)t.x, (int32_t)t.y, (int32_t)t.z, (int32_t)t.w};
+                // columns past the digits repeat the last one; nobody reads them
+                b[m] = *reinterpret_cast<const i4v*>(tab + p * kSuperBytes + ((m * 4 + g) * kDigits + min(r, kDigits - 1)) * 16);
+                sums = __builtin_amdgcn_mfma_i32_16x16x64_i8(ones, b[m], sums, 0, 0, 0);
+            }
+            const int wi = ((seg + p * kSuper) >> 3) + 4 * g;
+            const bool crosses = !NARROW && ((seg + (p + 1) * kSuper) >> 3) > kw && (kw & 3) != 0;   // wave-uniform
+#pragma unroll
+            for (int t = 0; t < RT; ++t) {
+                u4 w = wq[t][i];
+                if (crosses) {
+                    const int sh = wi - min(wi, kw - 4);     // 0..3, more where the lane is past the end
+                    const bool one = sh & 1, two = sh & 2;
+                    const u4 v = u4{one ? w.y : w.x, one ? w.z : w.y, one ? w.w : w.z, w.w};
+                    w = u4{two ? v.z : v.x, two ? v.w : v.y, v.z, v.w};
                 }
 #pragma unroll
-                for (int t = 0; t < RT; ++t) {
-                    const uint32_t w0 = m ? wq[t][i].z : wq[t][i].x, w1 = m ? wq[t][i].w : wq[t][i].y;
-                    const i4v a = {(int32_t)signed_nibbles(w0, 0), (int32_t)signed_nibbles(w0, 4),
-                                   (int32_t)signed_nibbles(w1, 0), (int32_t)signed_nibbles(w1, 4)};
-                    acc[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b, acc[t], 0, 0, 0);
+                for (int m = 0; m < 2; ++m) {
+                    const uint32_t w0 = m ? w.z : w.x, w1 = m ? w.w : w.y;
+                    const i4v a = {(int32_t)offset_nibbles(w0, 0), (int32_t)offset_nibbles(w0, 4),
+                                   (int32_t)offset_nibbles(w1, 0), (int32_t)offset_nibbles(w1, 4)};
+                    acc[t] = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, b[m], acc[t], 0, 0, 0);
                 }
             }
         }
     };
 
-    u4 xa0, xa1;
-    u4 wq0[RT][kPerWave], wq1[RT][kPerWave];
-    if (K > 0) issue(0, xa0, wq0);
-    for (int seg = 0; seg < K; seg += 2 * kSeg) {
-        __syncthreads();                                     // earlier table reads are done
-        build(seg, xa0);
-        __syncthreads();
-        if (seg + kSeg < K) issue(seg + kSeg, xa1, wq1);
-        multiply(seg, wq0);
-        if (seg + kSeg >= K) break;
-        __syncthreads();
-        build(seg + kSeg, xa1);
-        __syncthreads();
-        if (seg + 2 * kSeg < K) issue(seg + 2 * kSeg, xa0, wq0);
-        multiply(seg + kSeg, wq1);
+    u4 xa0, wq0[RT][kPerWave];
+    if constexpr (MULTI) {
+        u4 xa1, wq1[RT][kPerWave];
+        issue(0, xa0, wq0);
+        issue(kSeg, xa1, wq1);
+        for (int seg = 0; seg < K; seg += 2 * kSeg) {
+            build(seg, xa0, table);
+            lds_barrier();                                   // also: every wave is done with the other table
+            multiply(seg, wq0, table);
+            issue(seg + 2 * kSeg, xa0, wq0);
+            if (seg + kSeg < K) build(seg + kSeg, xa1, table + kTable);
+            lds_barrier();
+            if (seg + kSeg < K) multiply(seg + kSeg, wq1, table + kTable);
+            issue(seg + 3 * kSeg, xa1, wq1);
+        }
+    } else if (K > 0) {
+        issue(0, xa0, wq0);
+        build(0, xa0, table);
+        lds_barrier();
+        multiply(0, wq0, table);
     }
 
     if (r < kDigits) {
 #pragma unroll
         for (int t = 0; t < RT; ++t)
 #pragma unroll
-            for (int i = 0; i < 4; ++i) part[wave][kRows * t + 4 * g + i][r] = acc[t][i];
+            for (int i = 0; i < 4; ++i) part[wave][kRows * t + 4 * g + i][r] = acc[t][i] - 8 * sums[i];
     }
     const bool any_nonfinite = __syncthreads_or(nonfinite);
     if (tid < ROWS && row0 + tid < N) {
@@ -337,21 +374,27 @@ extern "C" int w4a16_gemv(const int32_t* W, const uint16_t* A, const uint16_t* s
         return W4A16_ERR_INVALID;
     }
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    // Two row tiles per workgroup once that still gives every CU a workgroup (N = 14336, K = 4096:
-    // 448 workgroups, 10.8 -> 9.9 us); one otherwise, so a small N still keeps every CU busy.
+    // Two row tiles per workgroup on one long segment (2048 < K <= 4096) once that still gives every CU a
+    // workgroup (N = 14336, K = 4096: 8.87 us against 9.24); one otherwise (N = 20000, K = 2000: 7.63
+    // against 7.84; N = 28672, K = 8192: 31.2 against 32.6; N = 4096, K = 14336: 10.3 against 15.7).
     int dev = 0, cus = 256;
     if (hipGetDevice(&dev) == hipSuccess) {
         w4a16_device_limits lim;
         if (w4a16_query_device(dev, &lim) == W4A16_OK && lim.cu_count > 0) cus = lim.cu_count;
     }
-    const bool two = (N + 2 * kRows - 1) / (2 * kRows) >= cus;
-    const dim3 grid((unsigned)((N + (two ? 2 : 1) * kRows - 1) / ((two ? 2 : 1) * kRows)));
-    const bool wvec = reinterpret_cast<uintptr_t>(W) % 16 == 0 && K % 32 == 0;
+    const bool two = K > 2048 && K <= kSeg && (N + 2 * kRows - 1) / (2 * kRows) >= cus;
+    const int rt = two ? 2 : 1;
+    const dim3 grid((unsigned)((N + rt * kRows - 1) / (rt * kRows)));
+    const bool narrow = K < 32, multi = K > kSeg;
     const bool xvec = reinterpret_cast<uintptr_t>(A) % 16 == 0;
-    auto pick = [&](auto rt) {
-        constexpr int R = decltype(rt)::value;
-        return wvec ? (xvec ? gemv_kernel<true, true, R> : gemv_kernel<true, false, R>)
-                    : (xvec ? gemv_kernel<false, true, R> : gemv_kernel<false, false, R>);
+    auto pick = [&](auto rt_c) {
+        constexpr int R = decltype(rt_c)::value;
+        if constexpr (R == 2)
+            return xvec ? gemv_kernel<false, true, R, false> : gemv_kernel<false, false, R, false>;
+        else
+            return narrow  ? (xvec ? gemv_kernel<true, true, R, false> : gemv_kernel<true, false, R, false>)
+                   : multi ? (xvec ? gemv_kernel<false, true, R, true> : gemv_kernel<false, false, R, true>)
+                           : (xvec ? gemv_kernel<false, true, R, false> : gemv_kernel<false, false, R, false>);
     };
     auto kernel = two ? pick(std::integral_constant<int, 2>{}) : pick(std::integral_constant<int, 1>{});
     hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, st, reinterpret_cast<const uint32_t*>(W), A, sW, zW, C, (int)N,
