@@ -1,5 +1,6 @@
-"""prefill_group_kernel_shared (the tiles of kSharedTable, w4a16_internal.h): small-batch prefill whose
-producer waves dequantise into LDS fragments that other waves multiply.
+"""The alternative prefill tiles (w4a16_internal.h): prefill_group_kernel_shared (kSharedTable, ids 1..6),
+small-batch prefill whose producer waves dequantise into LDS fragments that other waves multiply, and
+prefill_padded_kernel (kPaddedCfg, ids 7..10), the wide tiles for K / 64 that their step does not divide.
 
 CPU: the planner's choice, and an emulation of the kernel's index math (weights -> fragments -> MFMA
 operands, x staging, stage walk over odd chunk counts and segments, every address in bounds) against
@@ -26,15 +27,17 @@ TILES = {1: (2, 1, 1, 1, 8), 2: (2, 2, 2, 1, 8), 3: (4, 1, 2, 1, 12), 4: (4, 2, 
     (17, 4096, 4096, 1), (32, 4096, 4096, 1), (33, 4096, 4096, 2), (64, 4096, 4096, 2), (65, 4096, 4096, 4),
     (32, 6144, 4096, 2), (32, 14336, 4096, 4), (48, 14336, 4096, 5), (64, 14336, 4096, 6), (192, 4096, 4096, 5),
     (24, 10240, 4096, 3 + 1), (16, 14352, 4096, 3), (5, 10256, 1024, 0), (32, 4096, 512, 0), (24, 28672, 4096, 0),
-    (512, 4096, 4096, 0), (32, 4096, 14336, 0), (1, 4112, 4160, 1), (37, 4112, 4160, 3), (256, 4112, 4160, 5),
-    (1, 28672, 14400, 3), (4096, 4112, 4160, 0)])
+    (512, 4096, 4096, 0), (32, 4096, 14336, 0), (1, 4112, 4160, 1), (37, 4112, 4160, 3), (256, 4112, 4160, 7),
+    (1, 28672, 14400, 3), (4096, 4112, 4160, 9), (1024, 4112, 4160, 9), (2048, 14336, 4160, 10), (513, 4112, 4160, 7),
+    (1024, 28672, 14400, 8), (513, 6144, 4224, 7), (256, 14336, 4224, 7), (2048, 14336, 4224, 0), (256, 28672, 14464, 9),
+    (64, 4112, 14464, 0), (2048, 28672, 8192, 0)])
 def test_planner_choice(lib, M, N, K, want):
     rc, p, err = plan(lib, M=M, N=N, K=K, G=64)
     assert rc == 0 and p.kernel >= 1, err
     assert p.decode_variant == want
     assert _check(lib, p) == 0
     if want:
-        p.decode_variant = 7                       # no such tile
+        p.decode_variant = 11                      # no such tile
         assert _check(lib, p) == 1
 
 
@@ -159,9 +162,33 @@ def test_shared_tiles_bitwise_equal(monkeypatch, tile, M, N, K, G):
     assert_close(y, ref_gemm(x, q, scales, G, key))
 
 
+# Padded steps: K / 64 from one chunk to one past whole steps of 2 and 4, one chain and segments (the last
+# one odd), tails in M and N.  The 128 x 512 tile (id 10) has no second accumulator set.
 @pytest.mark.gpu
-@pytest.mark.parametrize("M,N,K", [(37, 4112, 4160), (24, 4096, 4096)])
-def test_shared_tiles_rows_keep_to_themselves(M, N, K):
+@pytest.mark.parametrize("tile", [7, 8, 9, 10])
+@pytest.mark.parametrize("M,N,K,G", [(1, 16, 64, 64), (65, 528, 128, 128), (130, 272, 192, 64), (129, 1040, 320, 64),
+                                     (300, 2064, 384, 128), (64, 512, 448, 64), (513, 4112, 4160, 64),
+                                     (128, 256, 8128, 64), (100, 272, 8256, 64), (200, 528, 14400, 64),
+                                     (150, 144, 14464, 128)])
+def test_padded_tiles_bitwise_equal(monkeypatch, tile, M, N, K, G):
+    torch = torch_cuda()
+    import w4a16_opt
+    if tile == 10 and K > 8192:
+        pytest.skip("one K chain only")
+    x, q, scales, Wp, key = make_problem(M, N, K, G, seed=M + K)
+    want = gemm(Wp, x, scales, variant=4)
+    monkeypatch.setenv("W4A16_PREFILL_SHARED", str(tile))
+    info = w4a16_opt.plan_info(M, N, K, G)
+    print(f"padded tile {tile}: M={M} N={N} K={K} G={G} {info['kernel_name']}", flush=True)
+    assert info["decode_variant"] == tile and "prefill_padded_kernel" in info["kernel_name"], info
+    y = gemm(Wp, x, scales)
+    assert torch.equal(y, want)
+    assert_close(y, ref_gemm(x, q, scales, G, key))
+
+
+@pytest.mark.gpu
+@pytest.mark.parametrize("M,N,K", [(37, 4112, 4160), (24, 4096, 4096), (513, 4112, 4160)])
+def test_rows_keep_to_themselves(M, N, K):
     """Infinities and NaN in one token row stay in that row; the other rows keep their bits."""
     torch = torch_cuda()
     x, q, scales, Wp, key = make_problem(M, N, K, 64, seed=3)
@@ -175,3 +202,24 @@ def test_shared_tiles_rows_keep_to_themselves(M, N, K):
     v4 = gemm(Wp, x2, scales, variant=4)
     assert torch.equal(torch.isnan(y2), torch.isnan(v4)) and torch.equal(torch.isinf(y2), torch.isinf(v4))
     assert torch.isnan(y2[9]).all()
+
+
+def test_padded_kernels_leave_pending_loads_alone(tmp_path):
+    """The check of test_isa_hazards on the padded kernels: no instruction touches the register of an
+    in-flight asm load before its wait."""
+    import os
+    import subprocess
+    import sys
+    from tests import test_isa_hazards as hz
+    if not os.path.exists(hz.HIPCC):
+        pytest.skip("hipcc not available")
+    sys.path.insert(0, os.path.join(hz.ROOT, "w4a16-gemm_amd"))
+    import build
+    src = "w4a16_prefill_wide.hip"
+    flags = [f for f in build.compile_flags(src) if f != "-fPIC"]
+    out = tmp_path / "wide.s"
+    subprocess.run([hz.HIPCC, *flags, "-S", "--cuda-device-only", os.path.join(hz.CSRC, src), "-o", str(out)], check=True,
+                   stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL)
+    ks = {k: v for k, v in hz._kernels(out.read_text()).items() if "prefill_padded_kernel" in k}
+    assert len(ks) == 7, list(ks)
+    assert not {k: v[:5] for k, v in ((k, hz.check_kernel(v)) for k, v in ks.items()) if v}

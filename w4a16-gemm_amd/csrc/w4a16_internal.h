@@ -171,6 +171,31 @@ constexpr bool shared_shape_ok(int id, int M, int N, int K) {
     return id >= 1 && id <= kNumSharedTiles && K < (1 << 25) && shared_tiles(id, M, N) < ((int64_t)1 << 31);
 }
 
+// Wide tiles for K / 64 that their loop's step does not divide (prefill_padded_kernel), ids after the
+// shared tiles: the config of kPrefillTable whose tile each is.  Steps of two chunks with the long-K
+// segments (whose length is even), else of the config's depth.
+constexpr int kNumPadded = 4;
+constexpr int kPaddedCfg[kNumPadded] = {18, 20, 24, 23};
+constexpr int kNumAltTiles = kNumSharedTiles + kNumPadded;
+constexpr int padded_cfg(int id) { return id > kNumSharedTiles && id <= kNumAltTiles ? kPaddedCfg[id - kNumSharedTiles - 1] : 0; }
+constexpr int padded_id(int cfg) {
+    for (int i = 0; i < kNumPadded; ++i)
+        if (kPaddedCfg[i] == cfg) return kNumSharedTiles + 1 + i;
+    return 0;
+}
+constexpr int64_t padded_tiles(int cfg, int M, int N) {
+    return (((int64_t)M + kPrefillTable[cfg].bm - 1) / kPrefillTable[cfg].bm) *
+           (((int64_t)N + kPrefillTable[cfg].bn - 1) / kPrefillTable[cfg].bn);
+}
+constexpr bool padded_shape_ok(int cfg, int M, int N, int K) {
+    return cfg > 0 && prefill_wide_offsets_fit(cfg, K) && padded_tiles(cfg, M, N) < ((int64_t)1 << 31) &&
+           (prefill_segments(K / 64) == 1 || prefill_wide_segmentable(cfg));
+}
+// Whether alternative tile `id` of a prefill plan (its decode_variant) can run the shape.
+constexpr bool alt_shape_ok(int id, int M, int N, int K) {
+    return id <= kNumSharedTiles ? shared_shape_ok(id, M, N, K) : padded_shape_ok(padded_cfg(id), M, N, K);
+}
+
 // Decode kernel shapes.  A workgroup covers NBW n16 blocks (16*NBW output channels) with WAVES
 // waves splitting its K range.
 //   kind 0: decode_kernel         weights streamed into VGPRs, pipeline depth d chunks, any

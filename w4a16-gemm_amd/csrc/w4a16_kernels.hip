@@ -1599,6 +1599,8 @@ prefill_group_kernel_shared(const u4* Wp, const uint16_t* x, const uint16_t* sca
 // compiled with a different instruction-scheduling strategy.
 hipError_t launch_prefill_wide(int cfg, const w4a16_plan& p, const u4* Wp, const uint16_t* x, const uint16_t* s,
                                uint16_t* y, hipStream_t st);
+hipError_t launch_prefill_padded(int cfg, const w4a16_plan& p, const u4* Wp, const uint16_t* x, const uint16_t* s,
+                                 uint16_t* y, hipStream_t st);
 int prefill_wide_occupancy(int cfg);
 hipError_t prefill_wide_load_code(hipStream_t st);
 
@@ -1718,8 +1720,8 @@ static hipError_t launch_shared_id(const w4a16_plan& p, const u4* Wp, const uint
         groups_m, prefill_segment_chunks(p.K >> 6), grid, y);
 }
 
-static hipError_t launch_prefill_shared(const w4a16_plan& p, const u4* Wp, const uint16_t* x, const uint16_t* s,
-                                        uint16_t* y, hipStream_t st) {
+static hipError_t launch_prefill_alt(const w4a16_plan& p, const u4* Wp, const uint16_t* x, const uint16_t* s,
+                                     uint16_t* y, hipStream_t st) {
     switch (p.decode_variant) {
         case 1: return launch_shared_id<1>(p, Wp, x, s, y, st);
         case 2: return launch_shared_id<2>(p, Wp, x, s, y, st);
@@ -1727,7 +1729,7 @@ static hipError_t launch_prefill_shared(const w4a16_plan& p, const u4* Wp, const
         case 4: return launch_shared_id<4>(p, Wp, x, s, y, st);
         case 5: return launch_shared_id<5>(p, Wp, x, s, y, st);
         case 6: return launch_shared_id<6>(p, Wp, x, s, y, st);
-        default: return hipErrorInvalidValue;
+        default: return launch_prefill_padded(padded_cfg(p.decode_variant), p, Wp, x, s, y, st);
     }
 }
 
@@ -1922,7 +1924,7 @@ int check_plan(const w4a16_plan& p) {
     if (segs > 1 && ((int64_t)p.counter_slots < tiles ||
                      p.workspace_bytes < (uint64_t)segs * p.M * p.N * sizeof(float)))
         return W4A16_ERR_WORKSPACE;
-    if (p.decode_variant && !shared_shape_ok(p.decode_variant, p.M, p.N, p.K)) return W4A16_ERR_INVALID;
+    if (p.decode_variant && !alt_shape_ok(p.decode_variant, p.M, p.N, p.K)) return W4A16_ERR_INVALID;
     return W4A16_OK;
 }
 }  // namespace
@@ -1949,7 +1951,7 @@ extern "C" int w4a16_launch(const w4a16_plan* plan, const int32_t* Wp, const uin
         int* cnt = reinterpret_cast<int*>(counters);
         e = launch_decode(p, wp, x, scales, y, ws, cnt, st);
     } else if (p.decode_variant) {
-        e = launch_prefill_shared(p, wp, x, scales, y, st);
+        e = launch_prefill_alt(p, wp, x, scales, y, st);
     } else {
         switch (p.kernel) {
             case 1: e = launch_prefill<1>(p, wp, x, scales, y, reinterpret_cast<float*>(workspace), counters, st); break;

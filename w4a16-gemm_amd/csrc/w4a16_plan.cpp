@@ -226,40 +226,68 @@ int prefill_select(int M, int N, int K, const w4a16_device_limits& lim) {
     return best;
 }
 
-// The shared-dequantisation tile (kSharedTable) to run instead of the auto config, or 0.  Measured on
-// MI355X over N = 256..28672, K = 1024..14400, M = 1..1024 (graph-timed, weights from HBM):
-//  * one K chain (K <= 8192): the narrowest tile whose workgroups fit one per CU.  It beats the auto
-//    config on every such shape, e.g. K = 4096: N = 4096, M = 24 8.4 vs 11.9 us (token groups of 16),
-//    M = 64 10.5 vs 12.1, M = 96 13.5 vs 15.7, M = 192 15.7 vs 18.8, M = 256 18.1 vs 19.9; N = 14336,
-//    M = 32 14.8 vs 16.4, M = 48 17.3 vs 21.2; N = 6144, M = 128 17.9 vs 18.9; in two rounds it loses
-//    (N = 28672, M = 32: 26 vs 21.6).  Not below K = 1024, where the launch of its larger workgroups
-//    outweighs the shorter chain, and the 64-channel tile only from K = 2048 (N = 10256, M = 5,
-//    K = 1024: 5.16 vs 4.79).
-//  * longer K: the token groups run the segments on workgroups of their own and are as fast (K = 14336,
-//    N = 4096, M = 32: 18.2 vs 18.6); kept.
-//  * K / 64 odd: the ring, token-group and wide kernels do not take it, prefill_kernel does at
-//    ~0.8 us per chunk, so the cheapest tile by rounds x us (scaled with K) while that is below 1.1 us
-//    per chunk: N = 4112, K = 4160, M = 37 11.6 vs 60.8 us, M = 513 47 vs 72; N = 28672, K = 14400,
-//    M = 1 65 vs 229; at M = 1024, N = 4112, K = 4160 both take 88.
-int shared_select(int M, int N, int K, const w4a16_device_limits& lim) {
-    const int64_t cus = lim.cu_count > 0 ? lim.cu_count : 1;
+// Whether an alternative prefill tile (decode_variant of a prefill plan) fits the device and the shape.
+bool alt_fits(int id, int M, int N, int K, const w4a16_device_limits& lim) {
+    if (id < 1 || id > kNumAltTiles || !alt_shape_ok(id, M, N, K)) return false;
+    if (const int cfg = padded_cfg(id)) return prefill_occupancy(cfg, lim) > 0;
+    return shared_lds_bytes(id) <= lim.lds_bytes_per_block && shared_threads(id) <= lim.max_threads_per_block;
+}
+
+// Estimated microseconds of alternative tile `id` (fitted to the sweep described at alt_select).
+double alt_us(int id, int M, int N, int K, double cus) {
     const int KC = K / 64;
-    auto ok = [&](int id) {
-        return shared_shape_ok(id, M, N, K) && shared_lds_bytes(id) <= lim.lds_bytes_per_block &&
-               shared_threads(id) <= lim.max_threads_per_block;
-    };
-    if (KC % 2 == 0) {
-        if (prefill_segments(KC) > 1 || KC < 16) return 0;
+    const int cfg = padded_cfg(id);
+    if (!cfg) return std::ceil(shared_tiles(id, M, N) / cus) * (2.6 + (kSharedTable[id].us - 2.6) * KC / 64.0);
+    const double fill = padded_tiles(cfg, M, N) / cus;
+    const double rounds = std::ceil(fill);
+    const bool seg = prefill_segments(KC) > 1;
+    // us per chunk: 18 and 20 run two workgroups per CU (one alone, then per round), 24 and 23 one (an
+    // emptier round leaves more clock)
+    if (cfg == 18)
+        return KC * (rounds <= 1   ? 0.467
+                     : rounds <= 2 ? (seg ? 0.49 + 0.10 * fill : 0.51 + 0.135 * fill)
+                                   : (seg ? 0.345 : 0.37) * rounds);
+    if (cfg == 20)
+        return KC * (rounds <= 1 ? (seg ? 0.55 + 0.11 * fill : 0.62 + 0.17 * fill) : (seg ? 0.54 : 0.61) * rounds);
+    const double lo = cfg == 24 ? (seg ? 0.76 : 0.65) : 1.11, slope = cfg == 24 ? (seg ? 0.33 : 0.46) : 0.95;
+    const double whole = std::floor(fill), part = fill - whole;
+    return KC * (whole * (lo + 0.85 * slope) + (part > 0 ? lo + slope * part : 0));
+}
+
+// The alternative tile (kSharedTable, then kPaddedCfg) to run instead of the auto config `cfg`, or 0.
+// Measured on MI355X over N = 256..28672, K = 1024..14464, M = 1..2048 (graph-timed, weights from HBM):
+//  * K / 64 odd: the ring, token-group and wide kernels do not take it and prefill_kernel needs ~0.8 us
+//    per chunk and round, so the alternative with the lowest estimate: N = 4112, K = 4160, M = 37 11.6 us
+//    (shared) against 60.8, M = 1024 54.3 (padded 128 x 256) against 93.7; N = 28672, K = 14400, M = 1 65
+//    against 229, M = 1024 908 against 2100; N = 14336, K = 8128, M = 2048 434 against 724.
+//  * one K chain (K <= 8192), K / 64 even: the narrowest shared tile whose workgroups fit one per CU.
+//    It beats the auto config on every such shape, e.g. K = 4096: N = 4096, M = 24 8.4 vs 11.9 us (token
+//    groups of 16), M = 64 10.5 vs 12.1, M = 96 13.5 vs 15.7, M = 192 15.7 vs 18.8, M = 256 18.1 vs 19.9;
+//    N = 14336, M = 32 14.8 vs 16.4, M = 48 17.3 vs 21.2; N = 6144, M = 128 17.9 vs 18.9; in two rounds it
+//    loses (N = 28672, M = 32: 26 vs 21.6).  Not below K = 1024, where the launch of its larger workgroups
+//    outweighs the shorter chain, and the 64-channel tile only from K = 2048 (N = 10256, M = 5, K = 1024:
+//    5.16 vs 4.79).  The segments of longer K run on workgroups of their own in the token groups, which
+//    are as fast (K = 14336, N = 4096, M = 32: 18.2 vs 18.6); kept.
+//  * K / 64 = 2 mod 4: the four-chunk wide configs (18, 20, 22, 24) are out.  Where the auto rules are left
+//    with prefill_kernel, the lowest estimate (K = 4224: N = 6144, M = 513 47 vs 76; N = 14336, M = 256 49
+//    vs 78); where they are left with the 64-token groups on long K, a padded tile that is estimated
+//    faster (K = 14464, N = 28672, M = 256 252 vs 420; N = 14336, M = 256 149 vs 199).
+int alt_select(int M, int N, int K, int cfg, const w4a16_device_limits& lim) {
+    const double cus = lim.cu_count > 0 ? lim.cu_count : 1;
+    const int KC = K / 64;
+    const bool odd = KC % 2 != 0, seg = prefill_segments(KC) > 1;
+    if (!odd && !seg && KC >= 16)
         for (int id = 1; id <= kNumSharedTiles; ++id)
-            if (ok(id) && shared_tiles(id, M, N) <= cus) return id == 3 && KC < 32 ? 0 : id;
-        return 0;
-    }
+            if (alt_fits(id, M, N, K, lim) && shared_tiles(id, M, N) <= cus)
+                return id == 3 && KC < 32 ? 0 : id;
+    const bool classic = cfg >= 1 && kPrefillTable[cfg].kind == 0;
+    const bool groups = KC % 4 == 2 && seg && cfg == 13;
+    if (!odd && !(KC % 4 == 2 && classic) && !groups) return 0;
     int best = 0;
-    double best_us = 1.1 * KC;
-    for (int id = 1; id <= kNumSharedTiles; ++id) {
-        if (!ok(id)) continue;
-        const double rounds = (double)((shared_tiles(id, M, N) + cus - 1) / cus);
-        const double us = rounds * (2.6 + (kSharedTable[id].us - 2.6) * KC / 64.0);
+    double best_us = groups ? 0.95 * 0.00172 * KC * std::ceil(M / 64.0) * std::ceil(N / 128.0) : std::numeric_limits<double>::infinity();
+    for (int id = groups ? kNumSharedTiles + 1 : 1; id <= kNumAltTiles; ++id) {
+        if (!alt_fits(id, M, N, K, lim)) continue;
+        const double us = alt_us(id, M, N, K, cus);
         if (us < best_us) { best_us = us; best = id; }
     }
     return best;
@@ -502,22 +530,22 @@ extern "C" int w4a16_plan_create(const w4a16_problem* prob, int variant, const w
                          out.slab_chunks, splits, out.grid);
     } else {
         int cfg = v;                                          // 1..4 forced, or -1 = auto
-        int shared = 0;
+        int shared = 0;                                       // alternative tile (-1: by rule)
         if (cfg < 0) {
             const char* o = std::getenv("W4A16_PREFILL");
-            const char* so = std::getenv("W4A16_PREFILL_SHARED");     // tuning override: shared tile id, 0 = none
-            const int sid = so ? std::atoi(so) : -1;
-            if (sid > 0 && shared_shape_ok(sid, M, N, K) && shared_lds_bytes(sid) <= lim->lds_bytes_per_block &&
-                shared_threads(sid) <= lim->max_threads_per_block)
-                shared = sid;
-            else if (sid < 0 && !o)
-                shared = shared_select(M, N, K, *lim);
+            const char* so = std::getenv("W4A16_PREFILL_SHARED");     // tuning override: alternative tile id, 0 = none
+            shared = so ? std::atoi(so) : -1;
+            if (shared > 0 && !alt_fits(shared, M, N, K, *lim)) shared = 0;
             if (o) {   // tuning override: prefill config id
                 const int oc = std::atoi(o);
                 if (oc >= 1 && oc <= kNumPrefillTable && prefill_occupancy(oc, *lim) > 0 && prefill_shape_ok(oc, M, K)) cfg = oc;
             }
         }
-        if (cfg < 0) cfg = prefill_select(M, N, K, *lim);
+        if (cfg < 0) {
+            cfg = prefill_select(M, N, K, *lim);
+            if (shared < 0) shared = alt_select(M, N, K, cfg, *lim);
+        }
+        shared = std::max(shared, 0);
         if (!(cfg >= 1 && cfg <= kNumPrefillTable && prefill_occupancy(cfg, *lim) > 0))
             return fail(W4A16_ERR_NO_CONFIG, err, errlen,
                         "no prefill configuration fits (shared memory limit %d B, M=%d)", lim->lds_bytes_per_block, M);

@@ -62,12 +62,13 @@ namespace w4a16 {
 // SEG: K longer than one canonical segment (seg_chunks chunks, even): acc holds the running
 // segment and total the sum of the finished ones (total = p0, then total + p_s), closed after
 // every seg_chunks chunks of the two-chunk loop.
-template <int BM, int BN, int WAVES_M, int WAVES_N, int WPE, bool SEG, int R>
-__global__ void __launch_bounds__(WAVES_M * WAVES_N * 64) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
-prefill_wide_kernel(const u4* __restrict__ Wp, const uint16_t* __restrict__ x,
-                    const uint16_t* __restrict__ scales,
-                    int M, int N, int K, int gshift, int tiles_m, int group_m, int seg_chunks, int G,
-                    uint16_t* __restrict__ y) {
+// PAD: K / 64 not a multiple of R.  The loop walks whole steps of R chunks; chunks past the end are fed
+// as zero x rows and zero scales, so their MFMAs add (+-0) * 0 and leave every accumulator as it is
+// (sums of fp16 products are multiples of 2^-48, so an accumulator is never -0).
+template <int BM, int BN, int WAVES_M, int WAVES_N, bool SEG, int R, bool PAD>
+__device__ __forceinline__ void
+wide_tile(const u4* __restrict__ Wp, const uint16_t* __restrict__ x, const uint16_t* __restrict__ scales,
+          int M, int N, int K, int gshift, int tiles_m, int group_m, int seg_chunks, int G, uint16_t* __restrict__ y) {
     constexpr int NT = WAVES_M * WAVES_N * 64;
     constexpr int WM = BM / WAVES_M;
     constexpr int WN = BN / WAVES_N;
@@ -143,9 +144,13 @@ prefill_wide_kernel(const u4* __restrict__ Wp, const uint16_t* __restrict__ x,
 #pragma unroll
         for (int i = 0; i < SPT; ++i) xr[i] = gload_u4_sbase(xb, xoff[i]);
     };
-    auto store_x = [&](int buf, u4 (&xr)[SPT]) __attribute__((always_inline)) {
+    auto store_x = [&](int buf, u4 (&xr)[SPT], bool live) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < SPT; ++i) bind_after_wait(xr[i]);
+        if (PAD && !live) {
+#pragma unroll
+            for (int i = 0; i < SPT; ++i) xr[i] = u4{0u, 0u, 0u, 0u};
+        }
 #pragma unroll
         for (int i = 0; i < SPT; ++i) {
             const int sg = tid + i * NT;
@@ -191,10 +196,11 @@ prefill_wide_kernel(const u4* __restrict__ Wp, const uint16_t* __restrict__ x,
     // while the reads are in flight, then one wait and the 4 TM TN MFMAs (tp = 0 before tp = 1).
     // The buffer and every B-operand offset are compile-time constants carried in the ds_read
     // offset field (no address arithmetic per read).
-    auto compute = [&](auto buf, u4 (&w)[TN][2], uint32_t (&s)[TN]) __attribute__((always_inline)) {
+    auto compute = [&](auto buf, u4 (&w)[TN][2], uint32_t (&s)[TN], bool live) __attribute__((always_inline)) {
 #pragma unroll
         for (int q = 0; q < TN; ++q) {
             bind_after_wait(w[q][0]); bind_after_wait(w[q][1]); bind_after_wait(s[q]);
+            if constexpr (PAD) s[q] &= live ? 0xFFFFu : 0u;
         }
         static_for<0, 2>([&](auto hh) {
             constexpr int h = decltype(hh)::value;
@@ -236,7 +242,7 @@ prefill_wide_kernel(const u4* __restrict__ Wp, const uint16_t* __restrict__ x,
     // seg_chunks chunks (and at the end), a multiple of R (checked by the planner).
     load_x(0, xr[0]);
     asm volatile("s_waitcnt vmcnt(0)" ::: "memory");
-    store_x(0, xr[0]);
+    store_x(0, xr[0], true);
     static_for<1, R + 1>([&](auto j) {
         constexpr int J = decltype(j)::value;
         load_x(J, xr[J % R]);
@@ -248,10 +254,10 @@ prefill_wide_kernel(const u4* __restrict__ Wp, const uint16_t* __restrict__ x,
             constexpr int T = decltype(t)::value;
             const int c = kc + T;
             wait_vmcnt<WAIT_X>();
-            store_x((T + 1) & 1, xr[(T + 1) % R]);
+            store_x((T + 1) & 1, xr[(T + 1) % R], c + 1 < KC);
             load_x(c + 1 + R, xr[(T + 1) % R]);
             wait_vmcnt<WAIT_W>();
-            compute(std::integral_constant<int, T & 1>{}, wr[T], sr[T]);
+            compute(std::integral_constant<int, T & 1>{}, wr[T], sr[T], c < KC);
             load_w(c + R, wr[T], sr[T]);
             __syncthreads();
         });
@@ -309,6 +315,24 @@ prefill_wide_kernel(const u4* __restrict__ Wp, const uint16_t* __restrict__ x,
             }
         }
     }
+}
+
+template <int BM, int BN, int WAVES_M, int WAVES_N, int WPE, bool SEG, int R>
+__global__ void __launch_bounds__(WAVES_M * WAVES_N * 64) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
+prefill_wide_kernel(const u4* __restrict__ Wp, const uint16_t* __restrict__ x,
+                    const uint16_t* __restrict__ scales,
+                    int M, int N, int K, int gshift, int tiles_m, int group_m, int seg_chunks, int G,
+                    uint16_t* __restrict__ y) {
+    wide_tile<BM, BN, WAVES_M, WAVES_N, SEG, R, false>(Wp, x, scales, M, N, K, gshift, tiles_m, group_m, seg_chunks, G, y);
+}
+
+template <int BM, int BN, int WAVES_M, int WAVES_N, int WPE, bool SEG, int R>
+__global__ void __launch_bounds__(WAVES_M * WAVES_N * 64) __attribute__((amdgpu_waves_per_eu(WPE, WPE)))
+prefill_padded_kernel(const u4* __restrict__ Wp, const uint16_t* __restrict__ x,
+                      const uint16_t* __restrict__ scales,
+                      int M, int N, int K, int gshift, int tiles_m, int group_m, int seg_chunks, int G,
+                      uint16_t* __restrict__ y) {
+    wide_tile<BM, BN, WAVES_M, WAVES_N, SEG, R, true>(Wp, x, scales, M, N, K, gshift, tiles_m, group_m, seg_chunks, G, y);
 }
 
 // The same tiles software-pipelined across chunks, for the 32-channel wave tiles that run one wave
@@ -605,6 +629,39 @@ static hipError_t launch_wide(const w4a16_plan& p, const u4* Wp, const uint16_t*
         launch_wide_kernel<CFG, false>(p, Wp, x, s, y, st, gshift, tiles_m, group_m, seg_chunks);
     }
     return hipGetLastError();
+}
+
+template <int CFG>
+static hipError_t launch_padded(const w4a16_plan& p, const u4* Wp, const uint16_t* x, const uint16_t* s, uint16_t* y,
+                                hipStream_t st) {
+    constexpr PrefillTile c = kPrefillTable[CFG];
+    const int tiles_m = (p.M + c.bm - 1) / c.bm;
+    const int grid = (int)padded_tiles(CFG, p.M, p.N);
+    const int group_m = std::min(kWideGroupM, tiles_m);
+    const int gshift = p.G == 128 ? 1 : 0, KC = p.K >> 6, seg_chunks = prefill_segment_chunks(KC);
+    const dim3 threads(c.waves_m * c.waves_n * 64);
+    if (prefill_segments(KC) > 1) {
+        if constexpr (prefill_wide_segmentable(CFG))
+            hipLaunchKernelGGL((prefill_padded_kernel<c.bm, c.bn, c.waves_m, c.waves_n, c.wpe, true, 2>), dim3(grid), threads,
+                               0, st, Wp, x, s, p.M, p.N, p.K, gshift, tiles_m, group_m, seg_chunks, grid, y);
+        else
+            return hipErrorInvalidValue;
+    } else {
+        hipLaunchKernelGGL((prefill_padded_kernel<c.bm, c.bn, c.waves_m, c.waves_n, c.wpe, false, c.depth>), dim3(grid),
+                           threads, 0, st, Wp, x, s, p.M, p.N, p.K, gshift, tiles_m, group_m, seg_chunks, grid, y);
+    }
+    return hipGetLastError();
+}
+
+hipError_t launch_prefill_padded(int cfg, const w4a16_plan& p, const u4* Wp, const uint16_t* x, const uint16_t* s,
+                                 uint16_t* y, hipStream_t st) {
+    switch (cfg) {
+        case 18: return launch_padded<18>(p, Wp, x, s, y, st);
+        case 20: return launch_padded<20>(p, Wp, x, s, y, st);
+        case 23: return launch_padded<23>(p, Wp, x, s, y, st);
+        case 24: return launch_padded<24>(p, Wp, x, s, y, st);
+        default: return hipErrorInvalidValue;
+    }
 }
 
 // A kernel that does nothing.  The HIP runtime loads each unit's GPU code on the first launch of

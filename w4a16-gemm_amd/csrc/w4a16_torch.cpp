@@ -294,7 +294,12 @@ py::dict w4a16_plan_info(int64_t M, int64_t N, int64_t K, int64_t G, int64_t var
                                        : tmpl(kinds[c.kind], {c.nbw, c.waves, c.d});
     } else {
         const w4a16::PrefillTile& t = w4a16::kPrefillTable[plan.kernel];
-        if (plan.decode_variant) {
+        if (const int pc = w4a16::padded_cfg(plan.decode_variant)) {
+            const w4a16::PrefillTile& c = w4a16::kPrefillTable[pc];
+            const bool segs = w4a16::prefill_segments((int)(K / 64)) > 1;
+            const std::string n = tmpl("prefill_padded_kernel", {c.bm, c.bn, c.waves_m, c.waves_n, c.wpe}, segs ? "true" : "false");
+            d["kernel_name"] = n.substr(0, n.size() - 1) + ", " + std::to_string(segs ? 2 : c.depth) + ">";
+        } else if (plan.decode_variant) {
             const w4a16::SharedTile& h = w4a16::kSharedTable[plan.decode_variant];
             d["kernel_name"] = tmpl("prefill_group_kernel_shared", {h.nb, h.tm, h.cb, h.ct, h.np});
         } else if (t.kind == 2)
