@@ -44,6 +44,21 @@ __device__ __forceinline__ f4 mfma16x16x32(h8 a, h8 b, f4 c) {
     return __builtin_amdgcn_mfma_f32_16x16x32_f16(a, b, c, 0, 0, 0);
 }
 
+// Between a 16x16x32 MFMA and the first read of its result other than as an MFMA's C operand lie 8 wait
+// states, which the compiler has to insert (the hardware does not interlock).  ROCm 7.2's hazard
+// recogniser looks at each predecessor block once, on the path it meets first; where a loop or a switch
+// merges, that can be a longer way round to the same MFMA, and the short path is left with too few (seen
+// as half of the outputs wrong, by code alignment).  So a kernel whose chain ends at such a merge
+// settles its accumulators there.
+template <int N>
+__device__ __forceinline__ void mfma_settle(f4 (&acc)[N]) {
+#pragma unroll
+    for (int i = 1; i < N; ++i) asm volatile("" : "+v"(acc[i]));
+    asm volatile("s_nop 7" : "+v"(acc[0]));
+#pragma unroll
+    for (int i = 1; i < N; ++i) asm volatile("" : "+v"(acc[i]));
+}
+
 // v_mfma_f32_32x32x16_f16: lane l supplies A[l % 32][8 (l / 32) + i] and B[8 (l / 32) + i][l % 32]
 // (i = 0..7); D register i of lane l is D[8 (i / 4) + 4 (l / 32) + i % 4][l % 32].  Measured on
 // MI355X: one 16x16x32 MFMA over k-slots 0..31 equals two chained 16x16x16 MFMAs over slots

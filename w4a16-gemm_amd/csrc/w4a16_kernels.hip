@@ -789,6 +789,9 @@ decode_ring_kernel(const u4* __restrict__ Wp, const uint16_t* __restrict__ x,
 #endif
         });
     });
+    // Single-block tiles keep the accumulator in VGPRs, which the partial sums' LDS store reads next
+    // (wider ones move it out of AGPRs, where the compiler places its waits correctly).
+    if constexpr (NBW == 1) mfma_settle(acc);
 
 #ifdef W4A16_WAVE_STAMPS
     const uint32_t st_done = stamp_clock();
@@ -1540,15 +1543,13 @@ prefill_group_kernel_shared(const u4* Wp, const uint16_t* x, const uint16_t* sca
             for (int i = 0; i < CB; ++i) acc[j][i] = mfma16x16x32(fa[i], fb[j], acc[j][i]);
     };
     __builtin_amdgcn_s_setprio(2);
-    int ks = 0, es = min(seg_chunks, KC);
     int off = 0;
-    bool first = true;
-    while (ks < KC) {
-        lds_barrier();
-        const int left = es - ks;
-        const char* xr = xr0 + off;
-        const char* ar = ar0 + off;
-        if (left >= 2 * P) {
+    for (int ks = 0; ks < KC; ks += seg_chunks) {
+        int left = min(seg_chunks, KC - ks);
+        for (; left >= 2 * P; left -= 2 * P) {
+            lds_barrier();
+            const char* xr = xr0 + off;
+            const char* ar = ar0 + off;
             static_for<0, 4 * P>([&](auto i) {
                 constexpr int I = decltype(i)::value, c = I / 2, h = I & 1;
                 step(xr + c * XCH + h * 64, ar + (c >> 1) * 4096 + (c & 1) * 512 + h * 2048);
@@ -1558,26 +1559,27 @@ prefill_group_kernel_shared(const u4* Wp, const uint16_t* x, const uint16_t* sca
                 __builtin_amdgcn_sched_group_barrier(0x008, CB * CT, 0);
                 if constexpr (decltype(i)::value + D < 4 * P) __builtin_amdgcn_sched_group_barrier(0x100, CB + CT, 0);
             });
-        } else {
+            off = BUF - off;
+        }
+        if (left > 0) {
+            lds_barrier();
+            const char* xr = xr0 + off;
+            const char* ar = ar0 + off;
 #pragma unroll 1
             for (int c = 0; c < left; ++c) {
                 step(xr + c * XCH, ar + (c >> 1) * 4096 + (c & 1) * 512);
                 step(xr + c * XCH + 64, ar + (c >> 1) * 4096 + (c & 1) * 512 + 2048);
             }
+            off = BUF - off;
         }
-        off = BUF - off;
-        ks += 2 * P;
-        if (ks >= es) {
-            ks = es;
-            es = min(es + seg_chunks, KC);
 #pragma unroll
-            for (int t = 0; t < CT; ++t)
+        for (int t = 0; t < CT; ++t) {
+            mfma_settle(acc[t]);
 #pragma unroll
-                for (int b = 0; b < CB; ++b) {
-                    total[t][b] = first ? acc[t][b] : total[t][b] + acc[t][b];
-                    acc[t][b] = f4{0.f, 0.f, 0.f, 0.f};
-                }
-            first = false;
+            for (int b = 0; b < CB; ++b) {
+                total[t][b] = ks == 0 ? acc[t][b] : total[t][b] + acc[t][b];
+                acc[t][b] = f4{0.f, 0.f, 0.f, 0.f};
+            }
         }
     }
 
