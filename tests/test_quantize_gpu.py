@@ -153,3 +153,11 @@ def test_quantize_pack_rejects_bad_shapes():
         w4a16_opt.quantize_pack(torch.zeros(16, 128, device="cuda", dtype=torch.bfloat16), 64)
     Wp, s = w4a16_opt.quantize_pack(torch.zeros(0, 128, device="cuda", dtype=torch.float16), 64)
     assert Wp.numel() == 0 and tuple(s.shape) == (2, 0)
+
+
+@pytest.mark.parametrize("dtype", ["fp16", "fp32"])
+@pytest.mark.parametrize("N,K", [(16, 128), (48, 64), (16, 320), (80, 192), (1040, 1088)])
+def test_quantize_pack_workgroups_with_idle_waves(N, K, dtype):
+    """G = 64 tiles (N / 16 * K / 64) with and without an idle wave in the last workgroup."""
+    W = np.random.default_rng([N, K, 7]).standard_normal((N, K)) * 0.02
+    _check(W.astype(np.float16 if dtype == "fp16" else np.float32), 64)

@@ -28,8 +28,8 @@ __device__ __forceinline__ int code_pos(int k) {
     return (k >> 6) * 64 + 16 * ((k >> 1) & 3) + 4 * ((k >> 4) & 3) + 2 * ((k >> 3) & 1) + (k & 1);
 }
 
-// Workgroup = 64 threads on one (n16 block, quantisation group) tile of 16 rows x G columns.
-// Phase 1: thread t owns row r = t / 4 and, in load j, the V = 16 / sizeof(T) consecutive values
+// One wave per (n16 block, quantisation group) tile of 16 rows x G columns; the NW waves of a
+// workgroup take consecutive tiles and share nothing.  Phase 1: thread t of the wave owns row r = t / 4 and, in load j, the V = 16 / sizeof(T) consecutive values
 // at column 4Vj + V(t % 4) of the group (each load instruction reads 64 contiguous bytes of 16
 // rows).  The 4 threads of a row reduce their absolute maxima with two lane swaps; every one of
 // them derives the row's scale, quantises its values in registers and stores the code pairs into
@@ -45,8 +45,8 @@ __device__ __forceinline__ int code_pos(int k) {
 // are decided as the reference decides them; otherwise rint(y) == rint(fl(v/s)) and the fast code
 // is exact.  |rint(v / s)| <= 7 for finite inputs, so the reference's clamp to [-8, 7] is a no-op
 // on the fast path; the slow path applies it.
-template <typename T, int G>
-__global__ void __launch_bounds__(64)
+template <typename T, int G, int NW>
+__global__ void __launch_bounds__(64 * NW)
 quantize_pack_kernel(const T* __restrict__ W, int N, int K, int32_t* __restrict__ Wp,
                      uint16_t* __restrict__ scales) {
     constexpr int V = 16 / (int)sizeof(T);                   // values per 16-byte load
@@ -54,11 +54,15 @@ quantize_pack_kernel(const T* __restrict__ W, int N, int K, int32_t* __restrict_
     constexpr int S = G + 16;                                // LDS row stride (bytes)
     constexpr float kMagic = 8388616.0f;                     // 2^23 + 8
     constexpr float kTieBand = 0.5f - 0x1p-18f;
-    __shared__ __align__(16) uint8_t codes[16 * S];
-    const int t = threadIdx.x;
+    __shared__ __align__(16) uint8_t codes_of[NW][16 * S];
+    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    uint8_t* codes = codes_of[wave];
+    const int t = threadIdx.x & 63;
     const int groups = K / G;
-    const int nb = blockIdx.x / groups;
-    const int grp = blockIdx.x - nb * groups;
+    const int tile = blockIdx.x * NW + wave;
+    if (tile >= (N >> 4) * groups) return;                   // a whole wave; no barrier below
+    const int nb = tile / groups;
+    const int grp = tile - nb * groups;
     const int r = t >> 2;
     const int part = t & 3;
 
@@ -116,7 +120,10 @@ quantize_pack_kernel(const T* __restrict__ W, int N, int K, int32_t* __restrict_
             *reinterpret_cast<uint16_t*>(row + code_pos(k)) = (uint16_t)pair;
         }
     }
-    __syncthreads();
+    // The codes are this wave's own and its LDS operations stay in order: no barrier, only the order.
+    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
 
     if (t < G / 2) {
         const int cl = t >> 5;                               // 64-wide chunk within the group
@@ -137,11 +144,18 @@ quantize_pack_kernel(const T* __restrict__ W, int N, int K, int32_t* __restrict_
 
 template <typename T>
 static hipError_t launch_quantize(const void* W, int N, int K, int G, int32_t* Wp, uint16_t* s, hipStream_t st) {
-    const dim3 grid((unsigned)((N / 16) * (K / G)));
+    const unsigned tiles = (unsigned)((N / 16) * (K / G));
+    // At G = 64 a wave's tile is half as large, and starting a workgroup per tile is what bounds the
+    // kernel once W is large; two waves per workgroup halve those.  One and two, W from HBM (MI355X):
+    // fp16 14336 x 4096 29.7 and 28.0 us, fp32 6144 x 4096 22.6 and 21.2, fp32 14336 x 8192 101.3 and 94.1
+    // (5.2 -> 5.6 TB/s), level at fp16 28672 x 4096 (54.7, 54.6) and up to 4096 x 4096; four and eight are
+    // no better.  G = 128 keeps one: level with two (fp16 14336 x 4096 30.9 both), slower with four (31.7).
+    constexpr int NW = 2;
     if (G == 64)
-        hipLaunchKernelGGL((quantize_pack_kernel<T, 64>), grid, dim3(64), 0, st, (const T*)W, N, K, Wp, s);
+        hipLaunchKernelGGL((quantize_pack_kernel<T, 64, NW>), dim3((tiles + NW - 1) / NW), dim3(64 * NW), 0, st,
+                           (const T*)W, N, K, Wp, s);
     else
-        hipLaunchKernelGGL((quantize_pack_kernel<T, 128>), grid, dim3(64), 0, st, (const T*)W, N, K, Wp, s);
+        hipLaunchKernelGGL((quantize_pack_kernel<T, 128, 1>), dim3(tiles), dim3(64), 0, st, (const T*)W, N, K, Wp, s);
     return hipGetLastError();
 }
 
