@@ -1373,9 +1373,9 @@ __device__ __forceinline__ void lds_barrier() {
 // Compiler-tracked loads only.  The input pointers are not __restrict__: the compiler would move the
 // prefetches across the memory barriers to just before their use.
 // What bounds it: per stage the chain load wait - dequantisation - LDS - barrier; 2.6 us per launch plus
-// 0.19 us per pair at two blocks x 16 tokens (o, N = K = 4096, M = 24: 11.9 -> 8.4 us; without the
-// MFMAs 7.1, without x 7.0; the bare stream of the weights 5.4); ragged N = 4112, K = 4160 (65
-// chunks), M = 37: 60.8 us (prefill_kernel) -> 11.6.
+// 0.19 us per pair at two blocks x 16 tokens (o, N = K = 4096, M = 24: 11.9 -> 8.0 us; a version of 8.4
+// took 7.1 without the MFMAs, 7.0 without x; the bare stream of the weights takes 5.4); ragged N = 4112,
+// K = 4160 (65 chunks), M = 37: 60.6 us (prefill_kernel) -> 10.6.
 template <int NB, int TM, int CB, int CT, int NP>
 __global__ void __launch_bounds__((NP + NB * TM / (CB * CT)) * 64)
 prefill_group_kernel_shared(const u4* Wp, const uint16_t* x, const uint16_t* scales,
