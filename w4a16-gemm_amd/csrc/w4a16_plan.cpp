@@ -261,7 +261,7 @@ double alt_us(int id, int M, int N, int K, double cus) {
 //    (shared) against 60.8, M = 1024 54.3 (padded 128 x 256) against 93.7; N = 28672, K = 14400, M = 1 65
 //    against 229, M = 1024 908 against 2100; N = 14336, K = 8128, M = 2048 434 against 724.
 //  * one K chain (K <= 8192), K / 64 even: the narrowest shared tile whose workgroups fit one per CU.
-//    It beats the auto config on every such shape, e.g. K = 4096: N = 4096, M = 24 8.4 vs 11.9 us (token
+//    It beats the auto config on every such shape, e.g. K = 4096: N = 4096, M = 24 8.0 vs 11.9 us (token
 //    groups of 16), M = 64 10.5 vs 12.1, M = 96 13.5 vs 15.7, M = 192 15.7 vs 18.8, M = 256 18.1 vs 19.9;
 //    N = 14336, M = 32 14.8 vs 16.4, M = 48 17.3 vs 21.2; N = 6144, M = 128 17.9 vs 18.9; in two rounds it
 //    loses (N = 28672, M = 32: 26 vs 21.6).  Not below K = 1024, where the launch of its larger workgroups
