@@ -41,6 +41,20 @@ def test_planner_choice(lib, M, N, K, want):
         assert _check(lib, p) == 1
 
 
+@pytest.mark.parametrize("N", [256, 4112, 28672])
+@pytest.mark.parametrize("M", [17, 64, 512, 2048])
+def test_short_k_keeps_the_tiled_kernel(lib, M, N):
+    """The padded tiles lose to prefill_kernel on the shortest K (measured at alt_select)."""
+    one_round = -(-M // 64) * -(-N // 128) <= 256
+    for chunks in (1, 2, 3, 5, 6, 7):
+        rc, p, err = plan(lib, M=M, N=N, K=64 * chunks, G=64)
+        assert rc == 0, err
+        if chunks < 3 or (chunks < 6 and not one_round):
+            assert p.decode_variant == 0, chunks
+        elif chunks % 2:
+            assert p.kernel <= 4 and p.decode_variant > 0, chunks
+
+
 def test_forced_variants_and_small_devices_take_no_shared_tile(lib):
     for v in (1, 2, 3, 4):
         rc, p, err = plan(lib, M=32, N=4096, K=4096, G=128, variant=v)
