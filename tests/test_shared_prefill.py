@@ -55,6 +55,18 @@ def test_short_k_keeps_the_tiled_kernel(lib, M, N):
             assert p.kernel <= 4 and p.decode_variant > 0, chunks
 
 
+@pytest.mark.parametrize("M,N,want", [
+    (44, 3952, {16: 2, 18: 0, 20: 0, 22: 0, 24: 2, 26: 2, 64: 2, 128: 2}),           # tile 2: whole stages, or from 24
+    (704, 256, {32: 2, 36: 2, 128: 2}), (1024, 256, {28: 2, 32: 2, 34: 0, 52: 0, 128: 0}),   # and at most 22 groups
+    (67, 6272, {16: 0, 22: 0, 64: 0, 128: 0}), (97, 4880, {18: 5, 64: 5}), (1078, 480, {24: 5, 40: 5}),
+    (106, 5856, {16: 0, 18: 0, 20: 6, 22: 0, 24: 6, 26: 0, 28: 6, 64: 6}),
+    (24, 2048, {16: 1, 18: 1, 22: 1, 128: 1}), (79, 3328, {16: 4, 18: 4, 22: 4, 128: 4})])
+def test_shared_tiles_only_where_they_win(lib, M, N, want):
+    """One K chain, an even number of chunks: the lines of shared_wins, measured on either side."""
+    got = {chunks: plan(lib, M=M, N=N, K=64 * chunks, G=64)[1].decode_variant for chunks in want}
+    assert got == want
+
+
 def test_forced_variants_and_small_devices_take_no_shared_tile(lib):
     for v in (1, 2, 3, 4):
         rc, p, err = plan(lib, M=32, N=4096, K=4096, G=128, variant=v)

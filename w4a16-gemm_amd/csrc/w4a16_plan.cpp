@@ -254,6 +254,28 @@ double alt_us(int id, int M, int N, int K, double cus) {
     return KC * (whole * (lo + 0.85 * slope) + (part > 0 ? lo + slope * part : 0));
 }
 
+// Whether shared tile `id`, in one round, is faster than auto config `cfg` on one K chain of KC chunks (even,
+// at least 16).  Measured on MI355X as the tile's time over the auto config's, 2,800 points of N = 256..28672,
+// M = 1..2048:
+//  * 1 and 4: 0.65-0.91 and 0.74-0.98;
+//  * 2 walks stages of 8 chunks: 0.96-0.99 at 16, 1.00-1.08 at 18..22 (M = 44, N = 3952, K = 1152: 5.6 vs 5.2
+//    us), 0.73-0.99 from 24.  With more than 22 token groups each XCD's 32 tiles read nearly all of x, which
+//    past its 4 MB L2 they read from further away: N = 256, M = 768 up to 1.05, M = 1024 1.01-1.26 from K = 2304
+//    (K = 2816: 1.26), 0.95-0.97 up to K = 2048;
+//  * 3: 0.87-0.97 from 32, 0.94-1.08 below (N = 10256, M = 5, K = 1024: 5.16 vs 4.79 us);
+//  * 5: 0.74-0.95, but 0.95-1.10 where the other is groups of 16 tokens in at most two workgroups per CU (M = 67,
+//    N = 6272, K = 1152: 8.1 vs 7.4 us); from three the fullest CU sets their time (M = 1078, N = 480, K = 2560: 0.79);
+//  * 6 walks stages of 4: 1.00-1.05 at 16, 18, 22 and 26, 0.96-0.99 at 20 and 24, 0.92-1.00 from 28.
+bool shared_wins(int id, int M, int N, int KC, int cfg, double cus) {
+    switch (id) {
+        case 2: return (KC % 8 == 0 || KC >= 24) && (M <= 22 * 32 || KC <= 32);
+        case 3: return KC >= 32;
+        case 5: return !(cfg == 17 && std::ceil(M / 16.0) * std::ceil(N / 64.0) <= 2.0 * cus);
+        case 6: return KC >= 28 || (KC % 4 == 0 && KC >= 20);
+        default: return true;
+    }
+}
+
 // The alternative tile (kSharedTable, then kPaddedCfg) to run instead of the auto config `cfg`, or 0.
 // Measured on MI355X over N = 256..28672, K = 1024..14464, M = 1..2048 (graph-timed, weights from HBM):
 //  * K / 64 odd: the ring, token-group and wide kernels do not take it and prefill_kernel needs ~0.8 us
@@ -264,14 +286,13 @@ double alt_us(int id, int M, int N, int K, double cus) {
 //    tiles lose everywhere (they walk whole steps of four; N = 4112, M = 1024, K = 64 10.7 vs 6.3), with 3 to
 //    5 once 64 x 128 tiles exceed one per CU (K = 192: N = 4112, M = 1024 10.8 vs 8.9, M = 256 4.9 vs 5.4), at
 //    6 nowhere by more than 2% (695 points, N = 256..28672, M = 1..2048, K = 64..1344).
-//  * one K chain (K <= 8192), K / 64 even: the narrowest shared tile whose workgroups fit one per CU.
-//    It beats the auto config on every such shape, e.g. K = 4096: N = 4096, M = 24 8.0 vs 11.9 us (token
+//  * one K chain (K <= 8192), K / 64 even: the narrowest shared tile whose workgroups fit one per CU, where it
+//    is faster than the auto config, e.g. K = 4096: N = 4096, M = 24 8.0 vs 11.9 us (token
 //    groups of 16), M = 64 10.5 vs 12.1, M = 96 13.5 vs 15.7, M = 192 15.7 vs 18.8, M = 256 18.1 vs 19.9;
 //    N = 14336, M = 32 14.8 vs 16.4, M = 48 17.3 vs 21.2; N = 6144, M = 128 17.9 vs 18.9; in two rounds it
 //    loses (N = 28672, M = 32: 26 vs 21.6).  Not below K = 1024, where the launch of its larger workgroups
-//    outweighs the shorter chain, and the 64-channel tile only from K = 2048 (N = 10256, M = 5, K = 1024:
-//    5.16 vs 4.79).  The segments of longer K run on workgroups of their own in the token groups, which
-//    are as fast (K = 14336, N = 4096, M = 32: 18.2 vs 18.6); kept.
+//    outweighs the shorter chain; lines per tile at shared_wins.  The segments of longer K run on
+//    workgroups of their own in the token groups, which are as fast (K = 14336, N = 4096, M = 32: 18.2 vs 18.6); kept.
 //  * K / 64 = 2 mod 4: the four-chunk wide configs (18, 20, 22, 24) are out.  Where the auto rules are left
 //    with prefill_kernel, the lowest estimate (K = 4224: N = 6144, M = 513 47 vs 76; N = 14336, M = 256 49
 //    vs 78); where they are left with the 64-token groups on long K, a padded tile that is estimated
@@ -280,11 +301,11 @@ int alt_select(int M, int N, int K, int cfg, const w4a16_device_limits& lim) {
     const double cus = lim.cu_count > 0 ? lim.cu_count : 1;
     const int KC = K / 64;
     const bool odd = KC % 2 != 0, seg = prefill_segments(KC) > 1;
+    const bool classic = cfg >= 1 && kPrefillTable[cfg].kind == 0;
     if (!odd && !seg && KC >= 16)
         for (int id = 1; id <= kNumSharedTiles; ++id)
             if (alt_fits(id, M, N, K, lim) && shared_tiles(id, M, N) <= cus)
-                return id == 3 && KC < 32 ? 0 : id;
-    const bool classic = cfg >= 1 && kPrefillTable[cfg].kind == 0;
+                return classic || shared_wins(id, M, N, KC, cfg, cus) ? id : 0;
     const bool groups = KC % 4 == 2 && seg && cfg == 13;
     if (!odd && !(KC % 4 == 2 && classic) && !groups) return 0;
     if (KC < 3 || (KC < 6 && padded_tiles(18, M, N) > cus)) return 0;
