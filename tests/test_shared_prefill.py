@@ -30,7 +30,7 @@ TILES = {1: (2, 1, 1, 1, 8), 2: (2, 2, 2, 1, 8), 3: (4, 1, 2, 1, 12), 4: (4, 2, 
     (512, 4096, 4096, 0), (32, 4096, 14336, 0), (1, 4112, 4160, 1), (37, 4112, 4160, 3), (256, 4112, 4160, 7),
     (1, 28672, 14400, 3), (4096, 4112, 4160, 9), (1024, 4112, 4160, 9), (2048, 14336, 4160, 10), (513, 4112, 4160, 7),
     (1024, 28672, 14400, 8), (513, 6144, 4224, 7), (256, 14336, 4224, 7), (2048, 14336, 4224, 0), (256, 28672, 14464, 9),
-    (64, 4112, 14464, 0), (2048, 28672, 8192, 0)])
+    (64, 4112, 14464, 0), (134, 28544, 10880, 9), (271, 18304, 8576, 9), (2048, 28672, 8192, 0)])
 def test_planner_choice(lib, M, N, K, want):
     rc, p, err = plan(lib, M=M, N=N, K=K, G=64)
     assert rc == 0 and p.kernel >= 1, err

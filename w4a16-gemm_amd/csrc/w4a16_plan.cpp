@@ -242,11 +242,13 @@ double alt_us(int id, int M, int N, int K, double cus) {
     const double rounds = std::ceil(fill);
     const bool seg = prefill_segments(KC) > 1;
     // us per chunk: 18 and 20 run two workgroups per CU (one alone, then per round), 24 and 23 one (an
-    // emptier round leaves more clock)
+    // emptier round leaves more clock).  Config 18's third round costs more than the others: 0.348-0.378 us a
+    // chunk and round against 0.329-0.342 at four and five (M = 134, N = 28544, K = 10880: 183 us, where padded
+    // 24 takes 171 and groups of 64 tokens 178).
     if (cfg == 18)
         return KC * (rounds <= 1   ? 0.467
                      : rounds <= 2 ? (seg ? 0.49 + 0.10 * fill : 0.51 + 0.135 * fill)
-                                   : (seg ? 0.345 : 0.37) * rounds);
+                                   : (!seg ? 0.37 : rounds == 3 ? 0.362 : 0.345) * rounds);
     if (cfg == 20)
         return KC * (rounds <= 1 ? (seg ? 0.55 + 0.11 * fill : 0.62 + 0.17 * fill) : (seg ? 0.54 : 0.61) * rounds);
     const double lo = cfg == 24 ? (seg ? 0.76 : 0.65) : 1.11, slope = cfg == 24 ? (seg ? 0.33 : 0.46) : 0.95;
