@@ -55,10 +55,37 @@ def test_row_tail_words_emulated(kw):
 @pytest.mark.gpu
 @pytest.mark.parametrize("N,K", [(1, 8), (17, 24), (16, 32), (33, 40), (15, 120), (16, 136), (31, 1016), (40, 2056),
                                  (8200, 2056), (8192, 4072), (9000, 4096), (50, 4104), (20, 8184), (5, 8192), (37, 8200),
-                                 (19, 12312), (3, 16400), (2, 131080)])
+                                 (19, 12312), (3, 16400), (2, 131080),
+                                 (4097, 32), (4112, 40), (4100, 1016), (4113, 1024), (4096, 1024), (4097, 1032), (8177, 2048),
+                                 (8200, 2040), (20490, 1160)])
 @pytest.mark.parametrize("w_off,a_off", [(0, 0), (1, 1), (3, 4)])
 def test_gemv_edges(N, K, w_off, a_off):
     print(f"gemv N={N} K={K} w_off={w_off} a_off={a_off}", flush=True)
     W, A, sW, zW = make_gemv(N, K, 11, special=True)
     C = _run(W, A, sW, zW, w_offset=w_off, a_offset=a_off).cpu().numpy()
     assert np.array_equal(bits(C), bits(c_oracle.gemv(W, A, sW, zW, exact=True)))
+
+
+def test_single_segment_kernels_load_only_what_they_multiply(tmp_path):
+    """A wave waits for every load it issued.  Up to K = 1024 and 2048 the longest segment gives a wave one and two
+    superchunks, so those instantiations request 1 and 2 pieces of 16 bytes per row tile, and one of A."""
+    import os
+    import re
+    import subprocess
+    import sys
+    from tests import test_isa_hazards as hz
+    if not os.path.exists(hz.HIPCC):
+        pytest.skip("hipcc not available")
+    sys.path.insert(0, os.path.join(hz.ROOT, "w4a16-gemm_amd"))
+    import build
+    flags = [f for f in build.compile_flags("w4a16_gemv.hip") if f != "-fPIC"]
+    out = tmp_path / "gemv.s"
+    subprocess.run([hz.HIPCC, *flags, "-S", "--cuda-device-only", os.path.join(hz.CSRC, "w4a16_gemv.hip"), "-o", str(out)],
+                   check=True, stdout=subprocess.DEVNULL, stderr=subprocess.DEVNULL)
+    seen = {}
+    for name, lines in hz._kernels(out.read_text()).items():
+        m = re.search(r"gemv_kernelILb0ELb1ELi(\d)ELb0ELi(\d)EE", name)      # 16-byte loads of A, one segment
+        if m:
+            text = "\n".join(lines)
+            seen[int(m[1]), int(m[2])] = text[:text.index("s_barrier")].count("global_load_dwordx4")
+    assert seen == {(rt, pw): 1 + rt * pw for rt, pw in ((1, 1), (1, 2), (1, 4), (2, 1), (2, 2))}

@@ -32,10 +32,11 @@
 // sums, so P_j = sum_k (wv + 8) L_j - 8 sum_k L_j (below 15 * 128 * 2^20 < 2^31 before the
 // subtraction).
 //
-// What bounds it: the launch and the first round trip at small N K (K = N = 4096: 4.7 us, 4.9 before this
-// loop), the weight stream at large (N = 28672, K = 8192: 31.2 us, 3.8 TB/s, 35.0 before).  Rows that are
-// not whole 16-byte units cost what others do: N = 9184, K = 888 4.6 us against 11.6 with 4-byte loads,
-// N = 20000, K = 2000 7.6 against 19.1; two segments in flight: N = 4096, K = 14336 10.3 against 13.9.
+// What bounds it: the launch and the first round trip at small N K (K = N = 4096: 4.5 us, 4.7 before this
+// loop), the weight stream at large (N = 28672, K = 8192: 28.4 us, 4.2 TB/s, 33.6 before).  Rows that are
+// not whole 16-byte units cost what others do: N = 9184, K = 888 3.9 us against 11.6 with 4-byte loads,
+// N = 20000, K = 2000 7.1 against 19.0; two segments in flight: N = 4096, K = 14336 9.7 against 13.3; short K,
+// only the loads that are multiplied: N = 8192, K = 512 3.3 against 4.0 (all timed in turn on one box).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
@@ -141,9 +142,12 @@ __device__ int nonfinite_class(const uint32_t* __restrict__ wrow, const uint16_t
 // pointers are not __restrict__, or it would move the loads down to their use.
 // RT: row tiles of 16 per workgroup.  Each digit-table B operand feeds RT + 1 MFMAs, so the A
 // conversion (done once per workgroup and segment) is shared by 16 RT rows.
+// PW: superchunks per wave that are loaded, at least those the longest segment gives a wave: 1 up to K = 1024,
+// 2 up to 2048.  A wave waits for all of its loads before it leaves, also for those that it does not multiply,
+// and always loading kPerWave cost N = 24576, K = 512 9.7 us against 4.7 with one and two row tiles (7.8 before this loop).
 typedef u4 u4_a4 __attribute__((aligned(4)));
 
-template <bool NARROW, bool XVEC, int RT, bool MULTI>
+template <bool NARROW, bool XVEC, int RT, bool MULTI, int PW>
 __global__ void __launch_bounds__(kThreads)
 gemv_kernel(const uint32_t* W, const uint16_t* A, const uint16_t* sW, const uint16_t* zW, uint16_t* C, int N, int K) {
     constexpr int ROWS = kRows * RT;
@@ -172,7 +176,7 @@ gemv_kernel(const uint32_t* W, const uint16_t* A, const uint16_t* sW, const uint
     };
     // Request the A values of this thread's 8-k unit and this wave's weights for segment `seg` (past
     // the end, MULTI: one cached address, unused).
-    auto issue = [&](int seg, u4& xa, u4 (&wq)[RT][kPerWave]) {
+    auto issue = [&](int seg, u4& xa, u4 (&wq)[RT][PW]) {
         const uint32_t live = !MULTI || seg < K ? 0xFFFFFFFFu : 0u;
         int nsc, per;
         shape(min(seg, K - 1), nsc, per);
@@ -187,7 +191,7 @@ gemv_kernel(const uint32_t* W, const uint16_t* A, const uint16_t* sW, const uint
             xa = u4{d[0], d[1], d[2], d[3]};
         }
 #pragma unroll
-        for (int i = 0; i < kPerWave; ++i) {
+        for (int i = 0; i < PW; ++i) {
             const int p = wave * per + min(i, per - 1);      // past the share: repeat its last one
             const int wi = ((seg + p * kSuper) >> 3) + 4 * g;   // first word of the lane's 32 weights
 #pragma unroll
@@ -246,12 +250,12 @@ gemv_kernel(const uint32_t* W, const uint16_t* A, const uint16_t* sW, const uint
 #pragma unroll
         for (int j = 0; j < kDigits; ++j) *reinterpret_cast<uint2*>(dst + 16 * j) = uint2{de[j], dd[j]};
     };
-    auto multiply = [&](int seg, const u4 (&wq)[RT][kPerWave], const uint8_t* tab) {
+    auto multiply = [&](int seg, const u4 (&wq)[RT][PW], const uint8_t* tab) {
         int nsc, per;
         shape(seg, nsc, per);
         const i4v ones = {0x01010101, 0x01010101, 0x01010101, 0x01010101};
 #pragma unroll
-        for (int i = 0; i < kPerWave; ++i) {
+        for (int i = 0; i < PW; ++i) {
             const int p = wave * per + i;
             if (i >= per || p >= nsc) break;
             i4v b[2];
@@ -283,9 +287,9 @@ gemv_kernel(const uint32_t* W, const uint16_t* A, const uint16_t* sW, const uint
         }
     };
 
-    u4 xa0, wq0[RT][kPerWave];
+    u4 xa0, wq0[RT][PW];
     if constexpr (MULTI) {
-        u4 xa1, wq1[RT][kPerWave];
+        u4 xa1, wq1[RT][PW];
         issue(0, xa0, wq0);
         issue(kSeg, xa1, wq1);
         for (int seg = 0; seg < K; seg += 2 * kSeg) {
@@ -374,29 +378,39 @@ extern "C" int w4a16_gemv(const int32_t* W, const uint16_t* A, const uint16_t* s
         return W4A16_ERR_INVALID;
     }
     hipStream_t st = reinterpret_cast<hipStream_t>(stream);
-    // Two row tiles per workgroup on one long segment (2048 < K <= 4096) once that still gives every CU a
-    // workgroup (N = 14336, K = 4096: 8.87 us against 9.24); one otherwise (N = 20000, K = 2000: 7.63
-    // against 7.84; N = 28672, K = 8192: 31.2 against 32.6; N = 4096, K = 14336: 10.3 against 15.7).
+    // Row tiles per workgroup, measured as the time of two over that of one (weights from HBM):
+    //  * K <= 1024: two once one tile each is more than a workgroup per CU; the digits of A and the launch are
+    //    most of the call (N = 8192: 0.89-0.98, N = 9000..12288 0.97-1.02, N = 28672 0.77-0.82; N = 4096 1.01-1.04);
+    //  * K <= 2048: two when that does not leave a CU a row tile more to do, or from six per CU (N = 7168, two
+    //    per CU 0.94-0.99; N = 14336, four 0.96-0.98; N = 24576, six 0.84-0.93; N = 9000, three 1.04-1.05);
+    //  * longer: one (N = 5000..8192 0.98-1.04, N = 9000..12288 1.14-1.17, N = 14336 1.03-1.05, N = 28672
+    //    1.03-1.11; at best 0.92, N = 24576, K = 2560).
     int dev = 0, cus = 256;
     if (hipGetDevice(&dev) == hipSuccess) {
         w4a16_device_limits lim;
         if (w4a16_query_device(dev, &lim) == W4A16_OK && lim.cu_count > 0) cus = lim.cu_count;
     }
-    const bool two = K > 2048 && K <= kSeg && (N + 2 * kRows - 1) / (2 * kRows) >= cus;
+    const bool narrow = K < 32, multi = K > kSeg;
+    const int64_t per_cu = ((N + kRows - 1) / kRows + cus - 1) / cus;
+    const bool two = !narrow && K <= kSeg / 2 && per_cu > 1 && (K <= kSeg / 4 || per_cu % 2 == 0 || per_cu > 5);
     const int rt = two ? 2 : 1;
     const dim3 grid((unsigned)((N + rt * kRows - 1) / (rt * kRows)));
-    const bool narrow = K < 32, multi = K > kSeg;
     const bool xvec = reinterpret_cast<uintptr_t>(A) % 16 == 0;
-    auto pick = [&](auto rt_c) {
-        constexpr int R = decltype(rt_c)::value;
-        if constexpr (R == 2)
-            return xvec ? gemv_kernel<false, true, R, false> : gemv_kernel<false, false, R, false>;
-        else
-            return narrow  ? (xvec ? gemv_kernel<true, true, R, false> : gemv_kernel<true, false, R, false>)
-                   : multi ? (xvec ? gemv_kernel<false, true, R, true> : gemv_kernel<false, false, R, true>)
-                           : (xvec ? gemv_kernel<false, true, R, false> : gemv_kernel<false, false, R, false>);
+    auto pick = [&](auto nx_c, auto rt_c, auto multi_c, auto pw_c) {
+        constexpr bool X = decltype(nx_c)::value, L = decltype(multi_c)::value;
+        constexpr int R = decltype(rt_c)::value, P = decltype(pw_c)::value;
+        return xvec ? gemv_kernel<X, true, R, L, P> : gemv_kernel<X, false, R, L, P>;
     };
-    auto kernel = two ? pick(std::integral_constant<int, 2>{}) : pick(std::integral_constant<int, 1>{});
+    constexpr std::integral_constant<int, 1> c1;
+    constexpr std::integral_constant<int, 2> c2;
+    constexpr std::integral_constant<int, kPerWave> c4;
+    constexpr std::false_type no;
+    constexpr std::true_type yes;
+    auto kernel = narrow          ? pick(yes, c1, no, c1)
+                  : K <= kSeg / 4 ? (two ? pick(no, c2, no, c1) : pick(no, c1, no, c1))
+                  : K <= kSeg / 2 ? (two ? pick(no, c2, no, c2) : pick(no, c1, no, c2))
+                  : multi         ? pick(no, c1, yes, c4)
+                                  : pick(no, c1, no, c4);
     hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, st, reinterpret_cast<const uint32_t*>(W), A, sW, zW, C, (int)N,
                        (int)K);
     const hipError_t e = hipGetLastError();
