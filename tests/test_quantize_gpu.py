@@ -161,3 +161,17 @@ def test_quantize_pack_workgroups_with_idle_waves(N, K, dtype):
     """G = 64 tiles (N / 16 * K / 64) with and without an idle wave in the last workgroup."""
     W = np.random.default_rng([N, K, 7]).standard_normal((N, K)) * 0.02
     _check(W.astype(np.float16 if dtype == "fp16" else np.float32), 64)
+
+
+@pytest.mark.parametrize("dtype,tiles", [("fp32", 4095), ("fp32", 4096), ("fp32", 4097), ("fp32", 16383), ("fp32", 16385),
+                                         ("fp32", 65536), ("fp32", 65537), ("fp16", 131072), ("fp16", 131073)])
+def test_quantize_pack_one_and_two_waves_per_workgroup(dtype, tiles):
+    """G = 64 on both sides of the line between one and two waves per workgroup, with and without an idle wave in
+    the last one.  The rows repeat every 13 tiles, and so do the oracle's."""
+    torch = torch_cuda()
+    rows = (np.random.default_rng(tiles).standard_normal((13 * 16, 64)) * 0.02).astype(np.float16 if dtype == "fp16" else np.float32)
+    Wp_ref, s_ref = _oracle(rows, 64)
+    W = torch.from_numpy(rows).cuda().repeat(-(-tiles // 13), 1)[:16 * tiles].contiguous()
+    Wp, s = _device(W, 64)
+    assert np.array_equal(Wp.reshape(tiles, -1), np.tile(Wp_ref.reshape(13, -1), (-(-tiles // 13), 1))[:tiles])
+    assert np.array_equal(s.view(np.uint16), np.tile(s_ref.view(np.uint16), (1, -(-tiles // 13)))[:, :16 * tiles])

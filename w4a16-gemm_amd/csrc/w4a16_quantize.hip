@@ -55,12 +55,12 @@ quantize_pack_kernel(const T* __restrict__ W, int N, int K, int32_t* __restrict_
     constexpr float kMagic = 8388616.0f;                     // 2^23 + 8
     constexpr float kTieBand = 0.5f - 0x1p-18f;
     __shared__ __align__(16) uint8_t codes_of[NW][16 * S];
-    const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
+    const int wave = NW > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x >> 6) : 0;
     uint8_t* codes = codes_of[wave];
-    const int t = threadIdx.x & 63;
+    const int t = NW > 1 ? threadIdx.x & 63 : threadIdx.x;
     const int groups = K / G;
-    const int tile = blockIdx.x * NW + wave;
-    if (tile >= (N >> 4) * groups) return;                   // a whole wave; no barrier below
+    const unsigned tile = blockIdx.x * NW + wave;
+    if (NW > 1 && tile >= (unsigned)((N >> 4) * groups)) return;         // a whole wave; no barrier below
     const int nb = tile / groups;
     const int grp = tile - nb * groups;
     const int r = t >> 2;
@@ -147,13 +147,19 @@ static hipError_t launch_quantize(const void* W, int N, int K, int G, int32_t* W
     const unsigned tiles = (unsigned)((N / 16) * (K / G));
     // At G = 64 a wave's tile is half as large, and starting a workgroup per tile is what bounds the
     // kernel once W is large; two waves per workgroup halve those.  One and two, W from HBM (MI355X):
-    // fp16 14336 x 4096 29.7 and 28.0 us, fp32 6144 x 4096 22.6 and 21.2, fp32 14336 x 8192 101.3 and 94.1
-    // (5.2 -> 5.6 TB/s), level at fp16 28672 x 4096 (54.7, 54.6) and up to 4096 x 4096; four and eight are
-    // no better.  G = 128 keeps one: level with two (fp16 14336 x 4096 30.9 both), slower with four (31.7).
-    constexpr int NW = 2;
-    if (G == 64)
-        hipLaunchKernelGGL((quantize_pack_kernel<T, 64, NW>), dim3((tiles + NW - 1) / NW), dim3(64 * NW), 0, st,
-                           (const T*)W, N, K, Wp, s);
+    //  * once W is larger than the 256 MB Infinity Cache: fp16 28672 x 8192 114.6-125.2 and 105.8-111.0 us,
+    //    fp32 14336 x 6144 77.7 and 76.2, 28672 x 8192 201.8 and 194.5;
+    //  * fp32 from 4096 to 16384 tiles: 4096 x 3072 12.4 and 11.7, 4096 x 4096 15.6 and 15.2.
+    // In between two win 0-6% on a W in HBM and lose 0-5% on one that the cache still holds (fp16 14336 x 8192
+    // 57.0 and 53.5, 56.5 and 58.2; fp32 8192 x 4096 29.7 and 29.1, 31.6 and 32.4); on smaller ones they lose
+    // (fp16 1024 x 1024 3.3 and 3.7, 4096 x 4096 11.2 and 11.7).  Four and eight are no better.
+    // G = 128 keeps one: fp16 level with two on large W and up to 23% faster on small, fp32 2% slower and 3% faster.
+    const uint64_t bytes = (uint64_t)N * K * sizeof(T);
+    const bool two = G == 64 && (bytes > 256u << 20 || (sizeof(T) == 4 && tiles >= 4096 && tiles <= 16384));
+    if (two)
+        hipLaunchKernelGGL((quantize_pack_kernel<T, 64, 2>), dim3((tiles + 1) / 2), dim3(128), 0, st, (const T*)W, N, K, Wp, s);
+    else if (G == 64)
+        hipLaunchKernelGGL((quantize_pack_kernel<T, 64, 1>), dim3(tiles), dim3(64), 0, st, (const T*)W, N, K, Wp, s);
     else
         hipLaunchKernelGGL((quantize_pack_kernel<T, 128, 1>), dim3(tiles), dim3(64), 0, st, (const T*)W, N, K, Wp, s);
     return hipGetLastError();
