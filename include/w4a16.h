@@ -86,8 +86,8 @@ typedef struct w4a16_plan {
     int32_t counter_slots;    /* ints of the counter buffer used (split-K fixup)         */
     int32_t decode_variant;   /* decode: kernel shape id (waves, n16 blocks per wave);    */
                               /* prefill: 0 = the config `kernel`, else the id of a tile  */
-                              /* that computes the same bits faster in its place (same    */
-                              /* scratch; grid and block stay those of `kernel`)          */
+                              /* that computes the same bits faster in its place and uses */
+                              /* no scratch; grid and block stay those of `kernel`        */
     uint64_t workspace_bytes; /* bytes of fp32 partials the launch needs (0 if none)     */
 } w4a16_plan;
 

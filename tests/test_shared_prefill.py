@@ -67,6 +67,21 @@ def test_shared_tiles_only_where_they_win(lib, M, N, want):
     assert got == want
 
 
+def test_alternative_tiles_ask_for_no_scratch(lib):
+    rng = np.random.default_rng(5)
+    long = 0
+    for _ in range(4000):
+        chunks = int(rng.integers(1, 480))
+        M, N = int(2 ** rng.uniform(4, 11)), 16 * int(2 ** rng.uniform(6, 10.8))
+        rc, p, err = plan(lib, M=M, N=N, K=64 * chunks, G=64)
+        assert rc == 0, err
+        if p.kernel >= 1 and p.decode_variant:
+            long += chunks > 128 and chunks % 2 == 0
+            assert (p.workspace_bytes, p.counter_slots, p.splits) == (0, 0, 1), (M, N, chunks, p.kernel, p.decode_variant)
+            assert _check(lib, p) == 0
+    assert long >= 10
+
+
 def test_forced_variants_and_small_devices_take_no_shared_tile(lib):
     for v in (1, 2, 3, 4):
         rc, p, err = plan(lib, M=32, N=4096, K=4096, G=128, variant=v)

@@ -226,6 +226,19 @@ int prefill_select(int M, int N, int K, const w4a16_device_limits& lim) {
     return best;
 }
 
+// A prefill config that needs no split-K scratch, sized by M: the wide tiles or the tiled kernel, which keep the
+// canonical K segments in registers; 0 when none fits.
+int scratch_free_cfg(int M, int K, const w4a16_device_limits& lim) {
+    static const int small_m[] = {2, 1, 4}, m64[] = {18, 3, 4}, m128[] = {20, 18, 4}, m256[] = {20, 7, 4},
+                     large_m[] = {24, 20, 7, 4};
+    const int* order = M <= 32 ? small_m : M <= 64 ? m64 : M <= 128 ? m128 : M <= 256 ? m256 : large_m;
+    const int n = order == large_m ? 4 : 3;
+    for (int i = 0; i < n; ++i)
+        if (kPrefillTable[order[i]].kind <= 1 && prefill_occupancy(order[i], lim) > 0 && prefill_shape_ok(order[i], M, K))
+            return order[i];
+    return 0;
+}
+
 // Whether an alternative prefill tile (decode_variant of a prefill plan) fits the device and the shape.
 bool alt_fits(int id, int M, int N, int K, const w4a16_device_limits& lim) {
     if (id < 1 || id > kNumAltTiles || !alt_shape_ok(id, M, N, K)) return false;
@@ -572,6 +585,11 @@ extern "C" int w4a16_plan_create(const w4a16_problem* prob, int variant, const w
         if (cfg < 0) {
             cfg = prefill_select(M, N, K, *lim);
             if (shared < 0) shared = alt_select(M, N, K, cfg, *lim);
+            // An alternative tile runs in place of `cfg` and splits nothing: no scratch for it.
+            if (shared > 0 && cfg > 0 && kPrefillTable[cfg].kind >= 2 && prefill_segments(K / 64) > 1) {
+                const int free = scratch_free_cfg(M, K, *lim);
+                if (free) cfg = free;
+            }
         }
         shared = std::max(shared, 0);
         if (!(cfg >= 1 && cfg <= kNumPrefillTable && prefill_occupancy(cfg, *lim) > 0))
@@ -599,23 +617,12 @@ extern "C" int w4a16_plan_create(const w4a16_problem* prob, int variant, const w
 
 namespace w4a16 {
 // A plan for the same prefill problem whose config needs no split-K scratch (every prefill config
-// gives the same bits): the wide tiles or the tiled kernel, which keep the canonical K segments
-// in registers, sized by M.  False when `in` is not a prefill plan.
+// gives the same bits).  False when `in` is not a prefill plan.
 bool prefill_plan_no_scratch(const w4a16_plan& in, const w4a16_device_limits& lim, w4a16_plan* out) {
     if (in.kernel < 1 || in.kernel > kNumPrefillTable) return false;
-    const int M = in.M, K = in.K;
-    static const int small_m[] = {2, 1, 4}, m64[] = {18, 3, 4}, m128[] = {20, 18, 4}, m256[] = {20, 7, 4},
-                     large_m[] = {24, 20, 7, 4};
-    const int* order = M <= 32 ? small_m : M <= 64 ? m64 : M <= 128 ? m128 : M <= 256 ? m256 : large_m;
-    const int n = order == large_m ? 4 : 3;
+    const int cfg = scratch_free_cfg(in.M, in.K, lim);
     *out = in;
-    for (int i = 0; i < n; ++i) {
-        const int cfg = order[i];
-        if (kPrefillTable[cfg].kind <= 1 && prefill_occupancy(cfg, lim) > 0 && prefill_shape_ok(cfg, M, K) &&
-            fill_prefill_plan(cfg, out))
-            return true;
-    }
-    return false;
+    return cfg > 0 && fill_prefill_plan(cfg, out);
 }
 }  // namespace w4a16
 
