@@ -82,6 +82,24 @@ def test_alternative_tiles_ask_for_no_scratch(lib):
     assert long >= 10
 
 
+def test_override_that_does_not_fit_is_ignored(lib, monkeypatch):
+    M, N, K = 256, 4112, 14400                                           # odd K / 64, several segments
+    auto = plan(lib, M=M, N=N, K=K, G=64)[1].decode_variant
+    assert auto > 0
+    for value, want in (("10", auto), ("11", auto), ("-3", auto), ("x", 0), ("0", 0), ("3", 3), ("9", 9)):
+        monkeypatch.setenv("W4A16_PREFILL_SHARED", value)                # id 10 has one K chain only
+        assert plan(lib, M=M, N=N, K=K, G=64)[1].decode_variant == want, value
+    monkeypatch.setenv("W4A16_PREFILL", "3")                             # both: the tile runs, based on config 3
+    p = plan(lib, M=M, N=N, K=K, G=64)[1]
+    assert (p.kernel, p.decode_variant) == (3, 9)
+    monkeypatch.setenv("W4A16_PREFILL_SHARED", "10")
+    p = plan(lib, M=M, N=N, K=K, G=64)[1]
+    assert (p.kernel, p.decode_variant) == (3, 0)
+    monkeypatch.delenv("W4A16_PREFILL_SHARED")
+    p = plan(lib, M=M, N=N, K=K, G=64)[1]
+    assert (p.kernel, p.decode_variant) == (3, 0)
+
+
 def test_forced_variants_and_small_devices_take_no_shared_tile(lib):
     for v in (1, 2, 3, 4):
         rc, p, err = plan(lib, M=32, N=4096, K=4096, G=128, variant=v)

@@ -574,9 +574,9 @@ extern "C" int w4a16_plan_create(const w4a16_problem* prob, int variant, const w
         int shared = 0;                                       // alternative tile (-1: by rule)
         if (cfg < 0) {
             const char* o = std::getenv("W4A16_PREFILL");
-            const char* so = std::getenv("W4A16_PREFILL_SHARED");     // tuning override: alternative tile id, 0 = none
+            const char* so = std::getenv("W4A16_PREFILL_SHARED");     // tuning override: alternative tile id that fits, 0 = none
             shared = so ? std::atoi(so) : -1;
-            if (shared > 0 && !alt_fits(shared, M, N, K, *lim)) shared = 0;
+            if (shared > 0 && !alt_fits(shared, M, N, K, *lim)) shared = -1;
             if (o) {   // tuning override: prefill config id
                 const int oc = std::atoi(o);
                 if (oc >= 1 && oc <= kNumPrefillTable && prefill_occupancy(oc, *lim) > 0 && prefill_shape_ok(oc, M, K)) cfg = oc;
