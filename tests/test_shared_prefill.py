@@ -216,6 +216,8 @@ def test_shared_tiles_bitwise_equal(monkeypatch, tile, M, N, K, G):
     info = w4a16_opt.plan_info(M, N, K, G)
     print(f"shared tile {tile}: M={M} N={N} K={K} G={G} {info['kernel_name']}", flush=True)
     assert info["decode_variant"] == tile and "prefill_group_kernel_shared" in info["kernel_name"], info
+    nb, tm, cb, ct, producers = TILES[tile]
+    assert (info["grid"], info["block"]) == (-(-M // (16 * tm)) * -(-(N // 16) // nb), 64 * (producers + nb * tm // (cb * ct)))
     y = gemm(Wp, x, scales)
     assert torch.equal(y, want)
     assert_close(y, ref_gemm(x, q, scales, G, key))
@@ -240,6 +242,8 @@ def test_padded_tiles_bitwise_equal(monkeypatch, tile, M, N, K, G):
     info = w4a16_opt.plan_info(M, N, K, G)
     print(f"padded tile {tile}: M={M} N={N} K={K} G={G} {info['kernel_name']}", flush=True)
     assert info["decode_variant"] == tile and "prefill_padded_kernel" in info["kernel_name"], info
+    bm, bn, waves = {7: (64, 128, 4), 8: (128, 128, 4), 9: (128, 256, 8), 10: (128, 512, 8)}[tile]
+    assert (info["grid"], info["block"], info["splits"]) == (-(-M // bm) * -(-N // bn), 64 * waves, 1)
     y = gemm(Wp, x, scales)
     assert torch.equal(y, want)
     assert_close(y, ref_gemm(x, q, scales, G, key))

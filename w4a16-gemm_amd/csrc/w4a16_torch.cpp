@@ -261,7 +261,8 @@ std::tuple<torch::Tensor, torch::Tensor> w4a16_quantize_pack_t(torch::Tensor W, 
     return {Wp, scales};
 }
 
-// Introspection used by the tests and the benchmark: the plan the op would launch.
+// Introspection used by the tests and the benchmark: the plan the op would launch (grid and block of the kernel
+// that runs, also where an alternative tile takes the place of the plan's config).
 py::dict w4a16_plan_info(int64_t M, int64_t N, int64_t K, int64_t G, int64_t variant, int64_t device) {
     w4a16_problem prob;
     prob.M = M; prob.N = N; prob.K = K;
@@ -299,9 +300,11 @@ py::dict w4a16_plan_info(int64_t M, int64_t N, int64_t K, int64_t G, int64_t var
             const bool segs = w4a16::prefill_segments((int)(K / 64)) > 1;
             const std::string n = tmpl("prefill_padded_kernel", {c.bm, c.bn, c.waves_m, c.waves_n, c.wpe}, segs ? "true" : "false");
             d["kernel_name"] = n.substr(0, n.size() - 1) + ", " + std::to_string(segs ? 2 : c.depth) + ">";
-        } else if (plan.decode_variant) {
-            const w4a16::SharedTile& h = w4a16::kSharedTable[plan.decode_variant];
+            d["grid"] = w4a16::padded_tiles(pc, (int)M, (int)N); d["block"] = w4a16::prefill_threads(pc);
+        } else if (const int id = plan.decode_variant) {
+            const w4a16::SharedTile& h = w4a16::kSharedTable[id];
             d["kernel_name"] = tmpl("prefill_group_kernel_shared", {h.nb, h.tm, h.cb, h.ct, h.np});
+            d["grid"] = w4a16::shared_tiles(id, (int)M, (int)N); d["block"] = w4a16::shared_threads(id);
         } else if (t.kind == 2)
             d["kernel_name"] = tmpl("prefill_stream_kernel", {t.bm / 16, t.depth});
         else if (t.kind == 3)
