@@ -100,6 +100,28 @@ def test_override_that_does_not_fit_is_ignored(lib, monkeypatch):
     assert (p.kernel, p.decode_variant) == (3, 0)
 
 
+def test_route_sweep_forces_every_alternative_tile(lib, monkeypatch):
+    import os
+    import sys
+    import types
+    from tests._helpers import PKG
+    monkeypatch.syspath_prepend(PKG)
+    import route_sweep
+
+    def info(M, N, K, G):
+        p = plan(lib, M=M, N=N, K=K, G=G)[1]
+        return {"kernel": p.kernel, "decode_variant": p.decode_variant, "splits": p.splits, "kernel_name": ""}
+
+    for var in route_sweep.OVERRIDES:                                    # stray values are cleared
+        monkeypatch.setenv(var, "2")
+    labels = [label for label, _, _ in route_sweep.forced_plans(types.SimpleNamespace(plan_info=info), 8, 4112, 4160, 64)]
+    assert labels == ["p1", "p2", "p3", "p4"] + [f"s{i}" for i in range(1, 11)]
+    labels = [label for label, _, _ in route_sweep.forced_plans(types.SimpleNamespace(plan_info=info), 8, 4096, 4096, 64)]
+    assert labels and all(label.startswith("d") for label in labels)
+    assert not any(var in os.environ for var in route_sweep.OVERRIDES)
+    sys.modules.pop("route_sweep", None)
+
+
 def test_forced_variants_and_small_devices_take_no_shared_tile(lib):
     for v in (1, 2, 3, 4):
         rc, p, err = plan(lib, M=32, N=4096, K=4096, G=128, variant=v)

@@ -2,8 +2,9 @@
 """Auto-route quality: the planner's choice against every forced config, per shape and batch size.
 
 For each (N, K, G) shape and M, times `w4a16_gemm(Wp, x, scales)` with the auto planner and with
-each prefill tile config forced through W4A16_PREFILL (M > 16) or each decode kernel shape and
-split count forced through W4A16_DECODE (M <= 16), and reports the auto config, the fastest
+each decode kernel shape and split count forced through W4A16_DECODE where the call takes the decode
+route, otherwise each prefill tile config forced through W4A16_PREFILL and each alternative tile
+forced through W4A16_PREFILL_SHARED, and reports the auto config, the fastest
 forced config and their ratio.  Timing is bench_gemm's: a HIP graph of calls over distinct weight
 copies (working set --target-mb), replayed untimed for --warm-ms first, median per call over
 --reps replays, the faster of two rounds (auto first in one, last in the other).  A forced
@@ -28,6 +29,8 @@ from bench_gemm import LLAMA3_8B, GraphTimer, load_weights  # noqa: E402
 SHAPES = [(name, n, k, 128) for name, (n, k) in LLAMA3_8B.items()] + [
     ("configs[2] gate", 14336, 4096, 64), ("configs[3] 70B gate_up", 28672, 8192, 128)]
 PREFILL_CONFIGS = range(1, 25)
+PREFILL_SHARED = range(1, 11)
+OVERRIDES = ("W4A16_PREFILL", "W4A16_PREFILL_SHARED", "W4A16_DECODE")
 DECODE_VARIANTS = range(0, 32)
 DECODE_SPLITS = (1, 2, 4)
 
@@ -46,24 +49,38 @@ def settled_timer(torch, calls, warm_ms: float):
     return timer
 
 
+def forced(settings: dict):
+    """Set the overrides to `settings` and nothing else."""
+    for var in OVERRIDES:
+        os.environ.pop(var, None)
+    os.environ.update(settings)
+
+
 def forced_plans(w4a16_opt, M, N, K, G):
-    """(label, env name, env value, kernel name) of every forced setting the planner accepts."""
+    """(label, overrides, kernel name) of every forced setting the planner accepts."""
+    forced({})
+    decode = w4a16_opt.plan_info(M, N, K, G)["kernel"] == 0
     out = []
-    if M <= 16:
+
+    def add(label, settings, want):
+        forced(settings)
+        info = w4a16_opt.plan_info(M, N, K, G)
+        if want(info):
+            out.append((label, settings, info["kernel_name"]))
+        forced({})
+
+    if decode:
         for v in DECODE_VARIANTS:
             for sp in DECODE_SPLITS:
-                os.environ["W4A16_DECODE"] = f"{v},{sp}"
-                info = w4a16_opt.plan_info(M, N, K, G)
-                del os.environ["W4A16_DECODE"]
-                if info["kernel"] == 0 and info["decode_variant"] == v and info["splits"] == sp:
-                    out.append((f"d{v}/{sp}", "W4A16_DECODE", f"{v},{sp}", info["kernel_name"]))
+                add(f"d{v}/{sp}", {"W4A16_DECODE": f"{v},{sp}"},
+                    lambda i: i["kernel"] == 0 and i["decode_variant"] == v and i["splits"] == sp)
     else:
+        # a table config alone: no alternative tile in its place
         for cfg in PREFILL_CONFIGS:
-            os.environ["W4A16_PREFILL"] = str(cfg)
-            info = w4a16_opt.plan_info(M, N, K, G)
-            del os.environ["W4A16_PREFILL"]
-            if info["kernel"] == cfg:
-                out.append((f"p{cfg}", "W4A16_PREFILL", str(cfg), info["kernel_name"]))
+            add(f"p{cfg}", {"W4A16_PREFILL": str(cfg), "W4A16_PREFILL_SHARED": "0"},
+                lambda i: i["kernel"] == cfg and i["decode_variant"] == 0)
+        for alt in PREFILL_SHARED:
+            add(f"s{alt}", {"W4A16_PREFILL_SHARED": str(alt)}, lambda i: i["kernel"] > 0 and i["decode_variant"] == alt)
     return out
 
 
@@ -84,8 +101,7 @@ def main(argv=None) -> int:
     import torch
     import w4a16_opt
     from w4a16_opt import w4a16_gemm
-    for var in ("W4A16_PREFILL", "W4A16_DECODE"):
-        os.environ.pop(var, None)
+    forced({})
 
     rows, dump = [], []
     for index, (name, N, K, G) in enumerate(shapes):
@@ -97,26 +113,21 @@ def main(argv=None) -> int:
             # Every setting is timed in each of two rounds (auto first in one, last in the
             # other) and keeps its faster median: a graph timed right after a switch of shapes
             # or clocks reads high.
-            forced = forced_plans(w4a16_opt, M, N, K, G)
+            settings = forced_plans(w4a16_opt, M, N, K, G)
             times = {}
-            for order in (["auto"] + forced, forced + ["auto"]):
-                for item in order:
-                    if item == "auto":
-                        us = settled_timer(torch, calls, args.warm_ms).per_call_us(args.reps)[0]
-                        times["auto"] = min(times.get("auto", us), us)
-                        continue
-                    label, var, value, kname = item
-                    os.environ[var] = value
+            for order in ([("auto", {}, "")] + settings, settings + [("auto", {}, "")]):
+                for label, overrides, _ in order:
+                    forced(overrides)
                     try:
                         us = settled_timer(torch, calls, args.warm_ms).per_call_us(args.reps)[0]
                     finally:
-                        del os.environ[var]
+                        forced({})
                     times[label] = min(times.get(label, us), us)
             auto_us = times["auto"]
-            best = min(((label, times[label], kname) for label, _, _, kname in forced), key=lambda b: b[1])
+            best = min(((label, times[label], kname) for label, _, kname in settings), key=lambda b: b[1])
             rows.append((name, N, K, G, M, auto["kernel_name"], auto_us, best))
             dump.append({"shape": name, "N": N, "K": K, "G": G, "M": M, "auto": auto["kernel_name"],
-                         "times_us": times, "kernels": {label: kname for label, _, _, kname in forced}})
+                         "times_us": times, "kernels": {label: kname for label, _, kname in settings}})
             print(f"{name} N={N} K={K} G={G} M={M}: auto {auto['kernel_name']} {auto_us:.2f} us; "
                   f"best forced {best[0]} {best[2]} {best[1]:.2f} us; auto/best {auto_us / best[1]:.3f}", flush=True)
             del x, calls
