@@ -183,134 +183,180 @@ def test_oracle_nonfinite_classes_agree_with_reference_order():
 
 SEG, SUPER, WAVES, DIGITS = 4096, 128, 8, 6
 THREADS, PER_WAVE = 64 * WAVES, SEG // SUPER // WAVES
-BIAS = 0x808080808080
 
 
-def biased_fixed(h):
-    """Vectorised biased_fixed() of the kernel: a * 2^24 + BIAS (X = 0 for inf / NaN)."""
-    h = h.astype(np.int64)
-    e, m = (h >> 10) & 31, h & 1023
-    mag = np.where(e == 0, m, (1024 | m) << np.maximum(e - 1, 0))
-    v = np.where(h & 0x8000, BIAS - mag, BIAS + mag)
-    return np.where(e == 31, BIAS, v)
+def split_digits(h):
+    """The table bytes that build() makes of fp16 bit patterns: split_fixed in float32 and the six balanced base-256
+    digits of its two halves, as digit_dwords takes them (inf and NaN count as 0)."""
+    h = np.where((h >> 10) & 31 == 31, 0, h).astype(np.uint16)
+    f = h.view(np.float16).astype(np.float32)
+    magic = np.float32(8388608 + 4227200)
+    m = (f + np.float32(0.00196)) + magic
+    lo = ((f - (m - magic)).astype(np.float64) * 2.0**24 + 8421504.0).astype(np.int64)      # one exact fma
+    hi = m.view(np.uint32).astype(np.int64)
+    low = [((lo >> (8 * j)) & 255) ^ 0x80 for j in range(3)]
+    high = [(hi & 255) ^ 0x80, ((hi >> 8) & 255) ^ 0x80, ((((hi >> 16) & 255) + 0x40) & 255) ^ 0x80]
+    return np.stack(low + high).astype(np.uint8)
 
 
-def test_digit_decomposition_of_every_fp16():
+def test_split_digits_of_every_fp16():
     h = np.arange(65536, dtype=np.uint16)
     finite = ((h >> 10) & 31) != 31
-    v = biased_fixed(h)
-    digits = np.stack([((v >> (8 * j)) & 0xFF) - 128 for j in range(DIGITS)])
-    assert digits.min() >= -128 and digits.max() <= 127
+    digits = split_digits(h).view(np.int8).astype(np.int64)
     X = sum(digits[j] * (256 ** j) for j in range(DIGITS))
     a = h.view(np.float16).astype(np.float64)
     assert np.array_equal(X[finite], (a[finite] * 2.0**24).astype(np.int64))
     assert (X[~finite] == 0).all()
 
 
-def test_signed_nibble_bytes():
-    w = np.arange(16, dtype=np.uint32)
-    words = (w[:, None] << (4 * np.arange(8, dtype=np.uint32))).astype(np.uint32)   # nibble v at position j
-    for shift in (0, 4):
-        u = ((words ^ np.uint32(0x88888888)) >> np.uint32(shift)) & np.uint32(0x0F0F0F0F)
-        s = (u + np.uint32(0x78787878)) ^ np.uint32(0x80808080)
-        sb = s.view(np.uint8).reshape(16, 8, 4).view(np.int8)
-        for j in range(8):
-            if (j & 1) * 4 != shift:
-                continue
-            for v in range(16):
-                want = np.zeros(4, np.int8)
-                want[j // 2] = v - 16 if v >= 8 else v
-                assert np.array_equal(sb[v, j], want), (shift, j, v)
+def offset_nibbles(w, shift):
+    return ((w >> shift) ^ 0x08080808) & 0x0F0F0F0F
 
 
-def emulate_gemv_kernel(W, A, N, K, wvec, rt=1):
-    """Digit sums P[n, j] of one launch, following gemv_kernel's indexing exactly: the A loads of
-    the table build, each lane's weight-load word indices (checked in bounds), the digit table,
-    the operand bytes and a 16x16x64 MFMA (A and B use the same k position for the same lane
-    group and byte, so any consistent hardware k order gives the same integer sums)."""
+def test_offset_nibble_bytes():
+    for j in range(8):
+        for v in range(16):
+            got = np.array([offset_nibbles((v << (4 * j)) | (0x77777777 & ~(15 << (4 * j))), 4 * (j & 1))], np.uint32)
+            want = np.full(4, 7 + 8)                                       # the other nibbles hold 7
+            want[j // 2] = (v - 16 if v >= 8 else v) + 8
+            assert np.array_equal(got.view(np.uint8), want), (j, v)
+
+
+def emulate_gemv_kernel(W, A, N, K, rt=1):
+    """Digit sums P[n, j] of one launch, following gemv_kernel's indexing exactly: the instantiation that the
+    dispatch takes for K (narrow rows, superchunks loaded per wave, one or two digit tables), the A loads of the
+    table build, each lane's weight-load word indices (checked in bounds) and its shift at the row's end, the order
+    of loads, tables and multiplications over the segments, the operand bytes and a 16x16x64 MFMA (A and B use the
+    same k position for the same lane group and byte, so any consistent hardware k order gives the same integer
+    sums), the digit sums and the int32 range of both."""
     kw = K // 8
+    narrow, multi = K < 32, K > SEG
+    pw = 1 if K <= SEG // 4 else 2 if K <= SEG // 2 else PER_WAVE
+    assert rt == 1 or (not narrow and K <= SEG // 2)
     Wu = W.view(np.uint32)
     h_all = A.view(np.uint16)
     P = np.zeros((N, DIGITS), dtype=object)
+
+    def shape(seg):
+        nsc = (min(SEG, K - seg) + SUPER - 1) // SUPER
+        return nsc, (nsc + WAVES - 1) // WAVES
+
     for row0 in range(0, N, 16 * rt):
         rows = [min(row0 + 16 * t + r, N - 1) for t in range(rt) for r in range(16)]
         acc = np.zeros((WAVES, 16 * rt, 16), dtype=np.int64)   # per wave: [row, column]
-        for seg in range(0, K, SEG):
-            seglen = min(SEG, K - seg)
-            nsc = (seglen + SUPER - 1) // SUPER
-            per = (nsc + WAVES - 1) // WAVES
-            table = np.full(SEG // SUPER * 768, 0xEE, dtype=np.uint8)   # poison: unwritten bytes
+        sums = np.zeros((WAVES, 16), dtype=np.int64)
+        tables = [np.full(SEG // SUPER * 768, 0xEE, dtype=np.uint8) for _ in range(2 if multi else 1)]
+        owner = [np.full(SEG // SUPER * 768, -1) for _ in tables]          # segment whose digits a byte holds
+
+        def issue(seg):
+            live = not multi or seg < K
+            _, per = shape(min(seg, K - 1))
+            xa = np.zeros((THREADS, 8), np.uint16)
             for tid in range(THREADS):
-                for u in (tid,):
-                    k0 = seg + 8 * u
-                    src = k0 if k0 < K else 0
-                    assert 0 <= src and (K == 0 or src + 8 <= K)
-                    if u >= nsc * 16:
-                        continue
-                    inside = k0 < K
-                    v = biased_fixed(h_all[src:src + 8]) if inside else np.full(8, BIAS, np.int64)
-                    p, rr = u >> 4, (u & 15) * 8
-                    gg, m, hh = rr >> 5, (rr >> 4) & 1, (rr >> 3) & 1
-                    base = p * 768 + ((m * 4 + gg) * DIGITS) * 16 + 8 * hh
-                    for j in range(DIGITS):
-                        for par in range(2):
-                            for i in range(4):
-                                byte = ((int(v[par + 2 * i]) >> (8 * j)) & 0xFF) ^ 0x80
-                                table[base + 16 * j + 4 * par + i] = byte
+                src = seg + 8 * tid if seg + 8 * tid < K else 0
+                assert src + 8 <= K
+                xa[tid] = h_all[src:src + 8]
+            wq = {}
             for wave in range(WAVES):
-                for i in range(PER_WAVE):
-                    p = wave * per + i
-                    p_load = wave * per + min(i, per - 1)          # loads past the share repeat
-                    lanes_words = {}
+                for i in range(pw):
+                    wi0 = (seg + (wave * per + min(i, per - 1)) * SUPER) >> 3
                     for g in range(4):
-                        for r in range(16 * rt):                   # row tile r // 16, lane row r % 16
-                            wi = ((seg + p_load * SUPER) >> 3) + 4 * g
-                            if wvec:
-                                idx = [wi + e for e in range(4)] if wi + 4 <= kw else [e for e in range(4)]
-                            else:
-                                idx = [wi + e if wi + e < kw else 0 for e in range(4)]
-                            assert all(0 <= x < kw for x in idx), (seg, p, g, idx)
-                            lanes_words[(r, g)] = [int(Wu[rows[r], x]) for x in idx]
+                        wi = wi0 + 4 * g
+                        for r in range(16 * rt):
+                            first = rows[r] * kw if live else row0 * kw      # past the end: the tile's first words
+                            idx = [min(wi + e, kw - 1) for e in range(4)] if narrow else \
+                                [(min(wi, kw - 4) if live else 0) + e for e in range(4)]
+                            assert all(0 <= x < kw for x in idx), (seg, wave, i, g, idx)
+                            wq[wave, i, r, g] = Wu.reshape(-1)[[first + x for x in idx]]
+            return xa, wq
+
+        def build(seg, xa, buf):
+            nsc, _ = shape(seg)
+            for u in range(min(THREADS, nsc * 16)):
+                d = split_digits(xa[u] if seg + 8 * u < K else np.zeros(8, np.uint16))
+                p, rr = u >> 4, (u & 15) * 8
+                gg, m, hh = rr >> 5, (rr >> 4) & 1, (rr >> 3) & 1
+                base = p * 768 + ((m * 4 + gg) * DIGITS) * 16 + 8 * hh
+                for j in range(DIGITS):
+                    at = slice(base + 16 * j, base + 16 * j + 8)
+                    tables[buf][at] = np.concatenate([d[j, 0::2], d[j, 1::2]])
+                    owner[buf][at] = seg
+
+        def multiply(seg, wq, buf):
+            nsc, per = shape(seg)
+            for wave in range(WAVES):
+                for i in range(pw):
+                    p = wave * per + i
                     if i >= per or p >= nsc:
                         break
-                    for m in range(2):
-                        Abytes = np.zeros((16 * rt, 4, 16), dtype=np.int64)  # [row r, group g, byte]
-                        Bbytes = np.zeros((16, 4, 16), dtype=np.int64)       # [column r, group g, byte]
-                        for g in range(4):
-                            for r in range(16 * rt):
-                                w = lanes_words[(r, g)]
-                                w0, w1 = (w[2], w[3]) if m else (w[0], w[1])
-                                dws = []
-                                for ww in (w0, w1):
-                                    for shift in (0, 4):
-                                        uu = ((ww ^ 0x88888888) >> shift) & 0x0F0F0F0F
-                                        dws.append(((uu + 0x78787878) ^ 0x80808080) & 0xFFFFFFFF)
-                                Abytes[r, g] = np.array(dws, dtype=np.uint32).view(np.int8)
-                                if r < DIGITS and r < 16:
-                                    off = p * 768 + ((m * 4 + g) * DIGITS + r) * 16
-                                    tb = table[off:off + 16]
-                                    assert not (tb == 0xEE).all(), "read of an unwritten table entry"
-                                    Bbytes[r, g] = tb.view(np.int8)
-                        acc[wave] += np.einsum("rgb,cgb->rc", Abytes, Bbytes)
+                    crosses = not narrow and (seg + (p + 1) * SUPER) >> 3 > kw and kw & 3
+                    a = np.zeros((2, 16 * rt, 4, 16), dtype=np.int64)      # [half m, row r, group g, byte]
+                    b = np.zeros((2, 16, 4, 16), dtype=np.int64)           # [half m, column r, group g, byte]
+                    for g in range(4):
+                        wi = ((seg + p * SUPER) >> 3) + 4 * g
+                        for r in range(16 * rt):
+                            w = [int(v) for v in wq[wave, i, r, g]]
+                            if crosses:
+                                sh = wi - min(wi, kw - 4)
+                                if sh & 1:
+                                    w = [w[1], w[2], w[3], w[3]]
+                                if sh & 2:
+                                    w = [w[2], w[3], w[2], w[3]]
+                            for m in range(2):
+                                dws = [offset_nibbles(ww, s) for ww in w[2 * m:2 * m + 2] for s in (0, 4)]
+                                a[m, r, g] = np.array(dws, dtype=np.uint32).view(np.uint8)
+                        for m in range(2):
+                            for r in range(16):
+                                off = p * 768 + ((m * 4 + g) * DIGITS + min(r, DIGITS - 1)) * 16
+                                assert (owner[buf][off:off + 16] == seg).all(), "another segment's digits"
+                                b[m, r, g] = tables[buf][off:off + 16].view(np.int8)
+                    assert a.min() >= 0 and a.max() <= 15
+                    acc[wave] += np.einsum("mrgb,mcgb->rc", a, b)
+                    sums[wave] += np.einsum("mcgb->c", b)
+                    assert max(np.abs(acc[wave]).max(), np.abs(8 * sums[wave]).max()) < 2**31
+
+        if multi:
+            sets = [issue(0), issue(SEG)]
+            for seg in range(0, K, 2 * SEG):
+                build(seg, sets[0][0], 0)
+                multiply(seg, sets[0][1], 0)
+                sets[0] = issue(seg + 2 * SEG)
+                if seg + SEG < K:
+                    build(seg + SEG, sets[1][0], 1)
+                    multiply(seg + SEG, sets[1][1], 1)
+                sets[1] = issue(seg + 3 * SEG)
+        else:
+            xa, wq = issue(0)
+            build(0, xa, 0)
+            multiply(0, wq, 0)
         for r in range(16 * rt):
             if row0 + r < N:
                 for j in range(DIGITS):
-                    P[row0 + r, j] = int(acc[:, r, j].sum())
+                    parts = acc[:, r, j] - 8 * sums[:, j]
+                    assert np.abs(parts).max() < 2**31 and np.abs(np.cumsum(parts)).max() < 2**31
+                    P[row0 + r, j] = int(parts.sum())
     return P
 
 
-@pytest.mark.parametrize("N,K,wvec,rt", [(16, 512, True, 1), (13, 4096 + 384, True, 1), (5, 1032, False, 1),
-                                         (3, 8, False, 1), (17, 160, True, 1), (40, 640, True, 2),
-                                         (29, 1032, False, 2), (32, 4096 + 128, True, 2)])
-def test_gemv_kernel_index_math_emulated(N, K, wvec, rt):
+@pytest.mark.parametrize("N,K,rt", [(3, 8, 1), (18, 24, 1), (5, 40, 1), (16, 512, 1), (17, 160, 1), (40, 640, 2), (33, 1016, 2),
+                                    (5, 1024, 1), (5, 1032, 1), (29, 1032, 2), (18, 2048, 2), (3, 2056, 1), (4, 3992, 1),
+                                    (4, 4096, 1), (3, 4104, 1), (13, 4096 + 384, 1), (2, 8192, 1), (3, 8200, 1), (2, 12312, 1),
+                                    (1, 16392, 1)])
+def test_gemv_kernel_index_math_emulated(N, K, rt):
     W, A, _, _ = make_gemv(N, K, 21, special=True)
-    P = emulate_gemv_kernel(W, A, N, K, wvec, rt)
+    P = emulate_gemv_kernel(W, A, N, K, rt)
     wv = signed_nibbles(W, K)
     X = [int(float(a) * 2**24) for a in A.astype(np.float64)]
     for n in range(N):
         total = sum(P[n, j] * 256 ** j for j in range(DIGITS))
         assert total == sum(int(w) * x for w, x in zip(wv[n], X)), n
-        assert all(abs(P[n, j]) < 2**31 for j in range(DIGITS))
+
+
+def test_digit_sums_fit_int32_at_the_largest_k():
+    """Offset weights (0..15) times digits (-128..127), 8 times the digit sum, and their difference (weights -8..7),
+    over all of K."""
+    K = 1 << 20
+    assert 15 * 128 * K < 2**31 and 8 * 128 * K < 2**31
 
 
 # ----------------------------------------------------------------------------- C ABI and binding (CPU)
