@@ -160,11 +160,18 @@ def isa(tmp_path_factory):
 
 
 def _kernels(text):
+    """Each kernel's whole body: up to the end of the function, past an s_endpgm of an early exit."""
     ks = {}
     for m in re.finditer(r"^(_ZN5w4a16\w+):", text, re.M):
-        end = text.find("s_endpgm", m.end())
+        end = text.find(".Lfunc_end", m.end())
         ks[m.group(1)] = text[m.end():end].splitlines()
     return ks
+
+
+def test_kernels_are_walked_to_their_end(isa):
+    """Some kernels end in more than one place; what follows the first s_endpgm is checked too."""
+    ends = [sum(t.strip().startswith("s_endpgm") for t in lines) for lines in _kernels(isa).values()]
+    assert min(ends) >= 1 and max(ends) >= 2
 
 
 def test_untracked_load_registers_untouched_until_waited(isa):
