@@ -58,6 +58,9 @@ MODERATE_CASE = ("gate_up", 14336, 4096, 128, 64)
 GRAPH_STEPS = 400                                            # longest timed region captured as one graph
 SIDE_STEPS, SIDE_WARMUP = 200, 20                            # timed and warm-up steps of the side legs
 GEMV_CASES = [("c1_shape", 4096, 4096), ("gate_up", 14336, 4096)]    # (name, N, K) of w4a16_ext.w4a16_gemv
+# The instantiations those calls run, as rocprofv3 names them (2048 < K <= 4096, A 16-byte aligned; fp16 W, G = 128).
+GEMV_KERNEL = "w4a16::(anonymous namespace)::gemv_kernel<false, true, 1, false, 4>"
+QUANT_KERNEL = "w4a16::quantize_pack_kernel<_Float16, 128, 1>"
 C1_CASE = ("c1", 4096, 4096, 1)                              # M=1, K=N=4096, G=128
 G = 128
 
@@ -329,10 +332,9 @@ def bench_gemv(torch, steps, warmup):
         us = ms * 1e3 / (steps * copies)
         gbs = gemv_bytes(N, K) / (us * 1e-6) / 1e9
         log(f"gemv {name} N={N} K={K}: {us:.2f} us  {gbs:.0f} GB/s")
-        rt = 2 if -(-N // 32) >= torch.cuda.get_device_properties(0).multi_processor_count else 1
         cases.append({"layer": name, "N": N, "K": K, "us": round(us, 3), "GBps": round(gbs, 1),
                       "frac_hbm": round(gbs / HBM_PEAK_GBS, 4), "copies": copies,
-                      "kernel": f"w4a16::(anonymous namespace)::gemv_kernel<true, true, {rt}>"})
+                      "kernel": GEMV_KERNEL})
         del Ws, g
     total_b = sum(gemv_bytes(c["N"], c["K"]) for c in cases)
     total_us = sum(c["us"] for c in cases)
@@ -608,7 +610,7 @@ def main(argv=None) -> int:
                "config": {"workload": f"quantize_pack of an fp16 [{N}, {K}] weight (BASELINE configs[3] weight), G={G}"},
                "roofline": {"bound": "hbm", "achieved": round(qr["GBs"], 1), "peak": HBM_PEAK_GBS, "unit": "GB/s",
                             "frac": round(qr["GBs"] / HBM_PEAK_GBS, 4),
-                            "kernel": "w4a16::quantize_pack_kernel<_Float16, 128>", "bytes_per_launch": quant_bytes(N, K)}}
+                            "kernel": QUANT_KERNEL, "bytes_per_launch": quant_bytes(N, K)}}
         tag_counters(out["roofline"], "quantize", [out["roofline"]["kernel"]], ["traffic"])
         if not a.no_cpu:
             out["cpu_baseline"] = cpu_baseline_quantize()

@@ -83,3 +83,22 @@ def test_small_sweep_on_gpu(tmp_path):
     y = w4a16_opt.w4a16_gemm(hip[0][0], x, hip[0][1]).float()
     ref = x.float() @ dense[0].float().t()
     assert (y - ref).abs().max().item() / ref.abs().max().item() < 2e-3
+
+
+def test_kernels_named_by_bench_and_by_the_counter_summary_exist():
+    """bench.py attaches counters to kernels by name, so a name that no longer exists would tag other code."""
+    import re
+    import shutil
+    lib = os.path.join(ROOT, "w4a16-gemm_amd", "libw4a16_hip.so")
+    if not os.path.exists(lib) or not shutil.which("c++filt"):
+        pytest.skip("library not built, or no c++filt")
+    if ROOT not in sys.path:
+        sys.path.insert(0, ROOT)
+    import bench
+    import pmc_summary
+    raw = set(re.findall(rb"_ZN5w4a16\w+", open(lib, "rb").read()))
+    names = {pmc_summary.kernel_name(n.decode()) for n in raw if b"kernel" in n}
+    assert {bench.QUANT_KERNEL, bench.GEMV_KERNEL} <= names
+    with open(os.path.join(ROOT, "profiles", "traffic.json")) as f:
+        measured = {k for entry in json.load(f).values() for k in entry["kernels"]}
+    assert measured <= names, measured - names

@@ -50,7 +50,8 @@ def kernel_name(raw: str) -> str:
 
 
 def read_runs(dirs):
-    """{kernel: {counter: [values]}} and {kernel: [durations ns]} over the runs' dispatches."""
+    """{kernel: {counter: [values]}} and {kernel: [durations ns]} over the runs' dispatches.  A kernel that a
+    workload launches at several shapes has an entry for each of its grids, named "kernel grid=work-items"."""
     vals = collections.defaultdict(lambda: collections.defaultdict(list))
     durs = collections.defaultdict(list)
     for d in dirs:
@@ -58,13 +59,15 @@ def read_runs(dirs):
         seen = set()
         with open(path, newline="") as f:
             for r in csv.DictReader(f):
-                name = kernel_name(r["Kernel_Name"])
+                name = (kernel_name(r["Kernel_Name"]), r["Grid_Size"])
                 vals[name][r["Counter_Name"]].append(float(r["Counter_Value"]))
                 key = (name, r["Dispatch_Id"])
                 if key not in seen:
                     seen.add(key)
                     durs[name].append(int(r["End_Timestamp"]) - int(r["Start_Timestamp"]))
-    return vals, durs
+    grids = collections.Counter(name for name, _ in vals)
+    label = {key: key[0] if grids[key[0]] == 1 else f"{key[0]} grid={key[1]}" for key in vals}
+    return {label[k]: v for k, v in vals.items()}, {label[k]: v for k, v in durs.items()}
 
 
 def median(xs):
@@ -98,7 +101,7 @@ def main(argv=None) -> int:
         kind, dirs = spec.split("=", 1)
         vals, durs = read_runs(dirs.split(","))
         kernels = sorted(k for k in vals if k.startswith("w4a16::"))
-        ent = {"kernels": kernels, "source": a.source, "per_kernel": {}}
+        ent = {"kernels": sorted({k.split(" grid=")[0] for k in kernels}), "source": a.source, "per_kernel": {}}
         traffic = []
         for k in kernels:
             c = vals[k]
