@@ -1372,8 +1372,8 @@ __device__ __forceinline__ void lds_barrier() {
 // load clamped data that is not multiplied or not stored; blocks past N repeat the last one.
 // Compiler-tracked loads only.  The input pointers are not __restrict__: the compiler would move the
 // prefetches across the memory barriers to just before their use.
-// What bounds it: per stage the chain load wait - dequantisation - LDS - barrier; 2.6 us per launch plus
-// 0.19 us per pair at two blocks x 16 tokens (o, N = K = 4096, M = 24: 11.9 -> 8.0 us; a version of 8.4
+// What bounds it: per stage the chain load wait - dequantisation - LDS - barrier; 2.2 us per launch plus
+// 0.18 us per pair at two blocks x 16 tokens (o, N = K = 4096, M = 24: 11.9 -> 8.0 us; a version of 8.4
 // took 7.1 without the MFMAs, 7.0 without x; the bare stream of the weights takes 5.4); ragged N = 4112,
 // K = 4160 (65 chunks), M = 37: 60.6 us (prefill_kernel) -> 10.6.
 template <int NB, int TM, int CB, int CT, int NP>

@@ -294,17 +294,17 @@ bool shared_wins(int id, int M, int N, int KC, int cfg, double cus) {
 // The alternative tile (kSharedTable, then kPaddedCfg) to run instead of the auto config `cfg`, or 0.
 // Measured on MI355X over N = 256..28672, K = 1024..14464, M = 1..2048 (graph-timed, weights from HBM):
 //  * K / 64 odd: the ring, token-group and wide kernels do not take it and prefill_kernel needs ~0.8 us
-//    per chunk and round, so from 6 chunks the alternative with the lowest estimate: N = 4112, K = 4160, M = 37 11.6 us
-//    (shared) against 60.8, M = 1024 54.3 (padded 128 x 256) against 93.7; N = 28672, K = 14400, M = 1 65
-//    against 229, M = 1024 908 against 2100; N = 14336, K = 8128, M = 2048 434 against 724.
+//    per chunk and round, so from 6 chunks the alternative with the lowest estimate: N = 4112, K = 4160, M = 37 10.7 us
+//    (shared) against 60.6, M = 1024 51.9 (padded 128 x 256) against 93.7; N = 28672, K = 14400, M = 1 66
+//    against 229, M = 1024 901 against 2100; N = 14336, K = 8128, M = 2048 432 against 724.
 //    Shorter K leaves little to overlap and the estimates have no fixed cost: with 1 or 2 chunks the padded
 //    tiles lose everywhere (they walk whole steps of four; N = 4112, M = 1024, K = 64 10.7 vs 6.3), with 3 to
 //    5 once 64 x 128 tiles exceed one per CU (K = 192: N = 4112, M = 1024 10.8 vs 8.9, M = 256 4.9 vs 5.4), at
 //    6 nowhere by more than 2% (695 points, N = 256..28672, M = 1..2048, K = 64..1344).
 //  * one K chain (K <= 8192), K / 64 even: the narrowest shared tile whose workgroups fit one per CU, where it
 //    is faster than the auto config, e.g. K = 4096: N = 4096, M = 24 8.0 vs 11.9 us (token
-//    groups of 16), M = 64 10.5 vs 12.1, M = 96 13.5 vs 15.7, M = 192 15.7 vs 18.8, M = 256 18.1 vs 19.9;
-//    N = 14336, M = 32 14.8 vs 16.4, M = 48 17.3 vs 21.2; N = 6144, M = 128 17.9 vs 18.9; in two rounds it
+//    groups of 16), M = 64 10.0 vs 12.1, M = 96 12.7 vs 15.7, M = 192 15.8 vs 18.8, M = 256 17.6 vs 19.9;
+//    N = 14336, M = 32 13.8 vs 16.4, M = 48 16.9 vs 21.2; N = 6144, M = 128 17.9 vs 18.9; in two rounds it
 //    loses (N = 28672, M = 32: 26 vs 21.6).  Not below K = 1024, where the launch of its larger workgroups
 //    outweighs the shorter chain; lines per tile at shared_wins.  The segments of longer K run on
 //    workgroups of their own in the token groups, which are as fast (K = 14336, N = 4096, M = 32: 18.2 vs 18.6); kept.
