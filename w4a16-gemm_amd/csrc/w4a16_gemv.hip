@@ -36,7 +36,7 @@
 // loop), the weight stream at large (N = 28672, K = 8192: 28.4 us, 4.2 TB/s, 33.6 before).  Rows that are
 // not whole 16-byte units cost what others do: N = 9184, K = 888 3.9 us against 11.6 with 4-byte loads,
 // N = 20000, K = 2000 7.1 against 19.0; two segments in flight: N = 4096, K = 14336 9.7 against 13.3; short K,
-// only the loads that are multiplied: N = 8192, K = 512 3.3 against 4.0 (all timed in turn on one box).
+// only the loads that are multiplied: N = 8192, K = 512 3.3 against 4.0 (both timed in turn).
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
