@@ -58,7 +58,7 @@ MODERATE_CASE = ("gate_up", 14336, 4096, 128, 64)
 GRAPH_STEPS = 400                                            # longest timed region captured as one graph
 SIDE_STEPS, SIDE_WARMUP = 200, 20                            # timed and warm-up steps of the side legs
 GEMV_CASES = [("c1_shape", 4096, 4096), ("gate_up", 14336, 4096)]    # (name, N, K) of w4a16_ext.w4a16_gemv
-# The instantiations those calls run, as rocprofv3 names them (2048 < K <= 4096, A 16-byte aligned; fp16 W, G = 128).
+# The instantiations those calls run, as rocprofv3 names them (3072 < K <= 4096, A 16-byte aligned; fp16 W, G = 128).
 GEMV_KERNEL = "w4a16::(anonymous namespace)::gemv_kernel<false, true, 1, false, 4>"
 QUANT_KERNEL = "w4a16::quantize_pack_kernel<_Float16, 128, 1>"
 C1_CASE = ("c1", 4096, 4096, 1)                              # M=1, K=N=4096, G=128

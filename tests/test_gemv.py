@@ -231,7 +231,7 @@ def emulate_gemv_kernel(W, A, N, K, rt=1):
     sums), the digit sums and the int32 range of both."""
     kw = K // 8
     narrow, multi = K < 32, K > SEG
-    pw = 1 if K <= SEG // 4 else 2 if K <= SEG // 2 else PER_WAVE
+    pw = 1 if K <= SEG // 4 else 2 if K <= SEG // 2 else 3 if K <= 3 * SEG // 4 else PER_WAVE
     assert rt == 1 or (not narrow and K <= SEG // 2)
     Wu = W.view(np.uint32)
     h_all = A.view(np.uint16)
@@ -339,7 +339,7 @@ def emulate_gemv_kernel(W, A, N, K, rt=1):
 
 
 @pytest.mark.parametrize("N,K,rt", [(3, 8, 1), (18, 24, 1), (5, 40, 1), (16, 512, 1), (17, 160, 1), (40, 640, 2), (33, 1016, 2),
-                                    (5, 1024, 1), (5, 1032, 1), (29, 1032, 2), (18, 2048, 2), (3, 2056, 1), (4, 3992, 1),
+                                    (5, 1024, 1), (5, 1032, 1), (29, 1032, 2), (18, 2048, 2), (3, 2056, 1), (2, 3072, 1), (3, 3080, 1), (4, 3992, 1),
                                     (4, 4096, 1), (3, 4104, 1), (13, 4096 + 384, 1), (2, 8192, 1), (3, 8200, 1), (2, 12312, 1),
                                     (1, 16392, 1)])
 def test_gemv_kernel_index_math_emulated(N, K, rt):

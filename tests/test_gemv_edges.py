@@ -57,7 +57,8 @@ def test_row_tail_words_emulated(kw):
                                  (8200, 2056), (8192, 4072), (9000, 4096), (50, 4104), (20, 8184), (5, 8192), (37, 8200),
                                  (19, 12312), (3, 16400), (2, 131080),
                                  (4097, 32), (4112, 40), (4100, 1016), (4113, 1024), (4096, 1024), (4097, 1032), (8177, 2048),
-                                 (8200, 2040), (20490, 1160)])
+                                 (8200, 2040), (20490, 1160),
+                                 (18, 3072), (33, 3080), (17, 3064)])
 @pytest.mark.parametrize("w_off,a_off", [(0, 0), (1, 1), (3, 4)])
 def test_gemv_edges(N, K, w_off, a_off):
     print(f"gemv N={N} K={K} w_off={w_off} a_off={a_off}", flush=True)
@@ -67,8 +68,8 @@ def test_gemv_edges(N, K, w_off, a_off):
 
 
 def test_single_segment_kernels_load_only_what_they_multiply(tmp_path):
-    """A wave waits for every load it issued.  Up to K = 1024 and 2048 the longest segment gives a wave one and two
-    superchunks, so those instantiations request 1 and 2 pieces of 16 bytes per row tile, and one of A."""
+    """A wave waits for every load it issued.  Up to K = 1024, 2048 and 3072 the longest segment gives a wave one, two and
+    three superchunks, so those instantiations request as many pieces of 16 bytes per row tile, and one of A."""
     import os
     import re
     import subprocess
@@ -88,4 +89,4 @@ def test_single_segment_kernels_load_only_what_they_multiply(tmp_path):
         if m:
             text = "\n".join(lines)
             seen[int(m[1]), int(m[2])] = text[:text.index("s_barrier")].count("global_load_dwordx4")
-    assert seen == {(rt, pw): 1 + rt * pw for rt, pw in ((1, 1), (1, 2), (1, 4), (2, 1), (2, 2))}
+    assert seen == {(rt, pw): 1 + rt * pw for rt, pw in ((1, 1), (1, 2), (1, 3), (1, 4), (2, 1), (2, 2))}

@@ -143,7 +143,7 @@ __device__ int nonfinite_class(const uint32_t* __restrict__ wrow, const uint16_t
 // RT: row tiles of 16 per workgroup.  Each digit-table B operand feeds RT + 1 MFMAs, so the A
 // conversion (done once per workgroup and segment) is shared by 16 RT rows.
 // PW: superchunks per wave that are loaded, at least those the longest segment gives a wave: 1 up to K = 1024,
-// 2 up to 2048.  A wave waits for all of its loads before it leaves, also for those that it does not multiply,
+// 2 up to 2048, 3 up to 3072.  A wave waits for all of its loads before it leaves, also for those that it does not multiply,
 // and always loading kPerWave cost N = 24576, K = 512 9.7 us against 4.7 with one and two row tiles (7.8 before this loop).
 typedef u4 u4_a4 __attribute__((aligned(4)));
 
@@ -383,8 +383,8 @@ extern "C" int w4a16_gemv(const int32_t* W, const uint16_t* A, const uint16_t* s
     //    most of the call (N = 8192: 0.89-0.98, N = 9000..12288 0.97-1.02, N = 28672 0.77-0.82; N = 4096 1.01-1.04);
     //  * K <= 2048: two when that does not leave a CU a row tile more to do, or from six per CU (N = 7168, two
     //    per CU 0.94-0.99; N = 14336, four 0.96-0.98; N = 24576, six 0.84-0.93; N = 9000, three 1.04-1.05);
-    //  * longer: one (N = 5000..8192 0.98-1.04, N = 9000..12288 1.14-1.17, N = 14336 1.03-1.05, N = 28672
-    //    1.03-1.11; at best 0.92, N = 24576, K = 2560).
+    //  * longer: one.  K <= 3072: N = 9000..12288 1.11-1.15, N = 14336, 16384 1.01-1.09, N = 28672 1.01-1.06, but
+    //    N = 22016..24576 and 40960 0.92-1.01; K <= 4096: 1.13-1.17, 1.03-1.06, 1.05-1.10 and 0.96-1.05.
     int dev = 0, cus = 256;
     if (hipGetDevice(&dev) == hipSuccess) {
         w4a16_device_limits lim;
@@ -403,14 +403,16 @@ extern "C" int w4a16_gemv(const int32_t* W, const uint16_t* A, const uint16_t* s
     };
     constexpr std::integral_constant<int, 1> c1;
     constexpr std::integral_constant<int, 2> c2;
+    constexpr std::integral_constant<int, 3> c3;
     constexpr std::integral_constant<int, kPerWave> c4;
     constexpr std::false_type no;
     constexpr std::true_type yes;
-    auto kernel = narrow          ? pick(yes, c1, no, c1)
-                  : K <= kSeg / 4 ? (two ? pick(no, c2, no, c1) : pick(no, c1, no, c1))
-                  : K <= kSeg / 2 ? (two ? pick(no, c2, no, c2) : pick(no, c1, no, c2))
-                  : multi         ? pick(no, c1, yes, c4)
-                                  : pick(no, c1, no, c4);
+    auto kernel = narrow              ? pick(yes, c1, no, c1)
+                  : K <= kSeg / 4     ? (two ? pick(no, c2, no, c1) : pick(no, c1, no, c1))
+                  : K <= kSeg / 2     ? (two ? pick(no, c2, no, c2) : pick(no, c1, no, c2))
+                  : K <= 3 * kSeg / 4 ? pick(no, c1, no, c3)
+                  : multi             ? pick(no, c1, yes, c4)
+                                      : pick(no, c1, no, c4);
     hipLaunchKernelGGL(kernel, grid, dim3(kThreads), 0, st, reinterpret_cast<const uint32_t*>(W), A, sW, zW, C, (int)N,
                        (int)K);
     const hipError_t e = hipGetLastError();
